@@ -43,7 +43,20 @@
 // garbage there cannot leak; pages past cdiv(seq_len, page_size) and pages not
 // named by the block table are never read.
 //
-// VALU path (fp32, and shapes the MFMA path does not take): lanes own 16-byte
+// MFMA path in fp32 (page_size % 16 == 0, head_dim in {64,128,256}): the same
+// segment on v_mfma_f32_16x16x4_f32, operands, weights and sums in fp32.
+//   S = K . Q^T     K restaged through LDS as above; a lane's 16 bytes are four
+//                   k steps.
+//   O^T += V^T P^T  V is loaded in the A operand's own layout (a lane's 16 bytes
+//                   are four output tiles of one token) and P is the score
+//                   tile's registers: neither touches LDS.
+// What bounds it: HBM on full batches, the longest sequence's workgroup on
+// ragged ones (uniform splits). Measured (us, VALU kernel -> this): 32/8/128
+// B=16 up to 4,096 tokens 384 -> 64, B=64 of 512 tokens 120 -> 47.6 (5.6 TB/s),
+// 32/1/128 B=16 up to 8,192 599 -> 43.6, 16/4/256 B=8 up to 4,096 200 -> 41.4,
+// 8/1/64 B=4 up to 512 62.7 -> 9.9.
+//
+// VALU path (shapes the MFMA paths do not take): lanes own 16-byte
 // slices of a token's head dims; dot products reduce across the lanes of a
 // token; each lane keeps an online softmax per query head and lanes merge by
 // the log-sum-exp rule at the end.
@@ -252,6 +265,27 @@ struct Mfma<BF16> {
   }
 };
 
+// fp32 products, four 16x16x4 MFMAs: element j of the operands is k step j, in
+// which lane l supplies A[row l % 16][k = l / 16] and B[k = l / 16][col l % 16].
+// Which four values of the contraction a step takes is free as long as A and B
+// agree, so both operands keep the 16-bit ones' shape (a lane holds 16
+// consecutive bytes of its row).
+template <>
+struct Mfma<F32> {
+  static __device__ __forceinline__ f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
+    const f32x4 av = __builtin_bit_cast(f32x4, a), bv = __builtin_bit_cast(f32x4, b);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j], bv[j], c, 0, 0, 0);
+    return c;
+  }
+};
+
+// Chunks of head_dim D that Q and K hold per lane: 16 bytes of every 64.
+template <typename E, int D>
+constexpr int qk_chunks() {
+  return D * E::kBytes / 64;
+}
+
 // O^T += V^T (P_hi + P_lo)^T over one 16-token block in one 16x16x32 product.
 // The softmax weights P are fp32; one 16-bit value keeps 8 (bf16) or 11
 // (fp16) of their bits, which left outputs near zero several ulps from the
@@ -281,15 +315,16 @@ constexpr int kDmaStages = 2;
 // LDS bytes the MFMA kernel needs: the per-wave K and V staging tiles during
 // the main loop, reused for the cross-wave merge afterwards (every wave's
 // output tiles, 16 bytes per lane each, and its running max and normaliser).
-template <int D, int NT, int W = kWaves, bool DMA = false, int NSD = kDmaStages>
+template <int D, int NT, int W = kWaves, bool DMA = false, int NSD = kDmaStages, int EB = 2>
 struct MfmaLds {
   // Register pipeline (DMA false): one block per wave staged at a time. Row
   // strides of a staged token: K's 8 elements (16 B) of pad put the 16 rows
   // one ds_read_b128 touches on distinct 16-byte bank groups; V's 16 elements
   // of pad put the 16 rows a transposing read touches on distinct 32-byte
   // bank groups two by two.
-  static constexpr int kKRow = D + 8;
-  static constexpr int kVRow = D + 16;
+  // fp32 (EB = 4) stages K alone, with the same 16 bytes of pad.
+  static constexpr int kKRow = D + 16 / EB;
+  static constexpr int kVRow = EB == 4 ? 0 : D + 16;
   static constexpr int kWaveStage = kBlock * (kKRow + kVRow);  // elements per wave
   // LDS pipeline (DMA true): NSD slots per wave, each one block's K
   // then V, 16 unpadded rows of D 16-bit elements with their 16-byte chunks
@@ -298,7 +333,7 @@ struct MfmaLds {
   static constexpr int kDmaSlotBytes = 2 * kBlock * D * 2;
   // ... followed by a block-table window: two halves of 64 entries.
   static constexpr int kDmaWaveBytes = NSD * kDmaSlotBytes + 2 * 64 * 4;
-  static constexpr int kStageBytes = DMA ? W * kDmaWaveBytes : W * kWaveStage * 2;
+  static constexpr int kStageBytes = DMA ? W * kDmaWaveBytes : W * kWaveStage * EB;
   static constexpr int kAccBytes = W * NT * (D / 16) * 64 * 16;
   static constexpr int kMlBytes = W * NT * 16 * 2 * 4;
   static constexpr int kBytes =
@@ -316,7 +351,7 @@ struct MfmaLds {
 // those keep registers.
 template <typename KVF, int D, int NT>
 constexpr bool dma_staged() {
-  return !std::is_same_v<KVF, Fp8E4M3> && D == 128 && NT == 1;
+  return KVF::kBytes == 2 && D == 128 && NT == 1;
 }
 
 // Register pipeline depth: blocks whose K and V are held in VGPRs at once
@@ -330,13 +365,25 @@ constexpr int mfma_stages() {
   return D <= 64 ? (NT == 2 ? 4 : 6) : 2;
 }
 
+// Waves of a one-unit uniform workgroup. fp32's MFMAs take several times the
+// cycles per cached byte that 16-bit ones do (a block of 16 tokens at head_dim
+// 128: 64 MFMAs of 32 cycles), and a workgroup has a CU to itself on most
+// batches (the planner aims at one per CU), so where the registers allow two
+// waves per SIMD one computes while the other loads. Measured, 4 -> 8 waves:
+// 32/8/128 B=16 up to 4,096 tokens 75.6 -> 64.3 us, 64/8/128 B=16 up to 2,048
+// 44.8 -> 35.8, 32/8/128 B=64 of 512 tokens equal.
+template <typename E, int D, int NT>
+constexpr int uniform_waves() {
+  return std::is_same_v<E, F32> && D <= 128 && NT == 1 ? 8 : kWaves;
+}
+
 // Occupancy floor (waves per SIMD) handed to the register allocator. With two
 // head tiles (GQA groups of 17-32) the default allocation lands just above
 // the two-wave budget; asking for two keeps the accumulators in VGPRs, no
 // spills. Single-tile kernels run best at the allocator's own choice.
-template <int D, int NT>
+template <int D, int NT, typename E = F16>
 constexpr int mfma_waves_per_eu() {
-  return NT == 2 ? 2 : 1;
+  return (NT == 2 && !std::is_same_v<E, F32>) || uniform_waves<E, D, NT>() == 8 ? 2 : 1;
 }
 
 // Row of q (and of the output) that local head hl of unit u reads.
@@ -379,14 +426,16 @@ __device__ __forceinline__ void fetch_args(const DecodeArgs& a) {
 // it waits for the sequence length. Nothing here uses the loaded values: the
 // compiler's wait for them lands where mfma_segment first does, before its
 // main loop.
+// fp32: dims 16c + 4grp .. +3 of chunk c.
 template <int NT, int KC>
 struct QFrag {
   u32x4 v[NT][KC];
 };
 
 template <typename E, int D, int NT>
-__device__ __forceinline__ void load_q(const DecodeArgs& a, const Unit& u, QFrag<NT, D / 32>& qf) {
+__device__ __forceinline__ void load_q(const DecodeArgs& a, const Unit& u, QFrag<NT, qk_chunks<E, D>()>& qf) {
   using S = typename E::S;
+  constexpr int EPC = 16 / E::kBytes;  // elements of a chunk per lane
   const int lane = __lane_id();
   const int row = lane & 15;
   const int grp = lane >> 4;
@@ -397,7 +446,9 @@ __device__ __forceinline__ void load_q(const DecodeArgs& a, const Unit& u, QFrag
     const int hl = h0 + 16 * t + row;
     const S* qh = q + q_row(a, u, hl < a.group ? hl : 0) * D;
 #pragma unroll
-    for (int c = 0; c < D / 32; ++c) qf.v[t][c] = *reinterpret_cast<const u32x4*>(qh + 32 * c + 8 * grp);
+    for (int c = 0; c < qk_chunks<E, D>(); ++c) {
+      qf.v[t][c] = *reinterpret_cast<const u32x4*>(qh + EPC * (4 * c + grp));
+    }
   }
 }
 
@@ -455,14 +506,15 @@ __device__ __forceinline__ void prefetch_window(const DecodeArgs& a, char* lds, 
 // loads for this segment (prefetch_window); LDS pipeline only.
 template <typename E, typename KVF, int D, int NT, int W = kWaves, int NSD = kDmaStages>
 __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, const Unit& u, const Dest& dst,
-                                             const int wave, const QFrag<NT, D / 32>* qpre = nullptr,
+                                             const int wave, const QFrag<NT, qk_chunks<E, D>()>* qpre = nullptr,
                                              const bool win_ready = false) {
   using S = typename E::S;
   using KS = typename KVF::S;          // cache storage type
   using M = Mfma<E>;
   constexpr bool KV8 = std::is_same_v<KVF, Fp8E4M3>;
+  constexpr bool FP32 = std::is_same_v<E, F32>;
   constexpr int KB = KVF::kBytes;      // cache bytes per element
-  constexpr int KC = D / 32;           // QK k-chunks
+  constexpr int KC = qk_chunks<E, D>();  // QK k-chunks
   constexpr int DT = D / 16;           // PV output tiles along head_dim
   constexpr int EPL = 16 / KB;         // cache elements per 16-byte lane load
   constexpr int LPT = D / EPL;         // lanes per token row in a load
@@ -470,7 +522,7 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
   constexpr int NL = kBlock / TPL;     // 16-byte loads per lane per block, each of K and V
   static_assert(TPL <= kBlock && kBlock % TPL == 0, "a load must stay inside its 16-token block");
   constexpr bool kDma = dma_staged<KVF, D, NT>();
-  using Lds = MfmaLds<D, NT, W, kDma, NSD>;
+  using Lds = MfmaLds<D, NT, W, kDma, NSD, E::kBytes>;
   constexpr int KROW = Lds::kKRow;
   constexpr int VROW = Lds::kVRow;
   constexpr int NS = mfma_stages<D, NT>();
@@ -528,12 +580,19 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
   // loads off a per-block wave-uniform base. Load c covers tokens
   // c*TPL .. c*TPL + TPL-1; lane l reads 16 bytes (EPL elements) of token
   // c*TPL + l/LPT, head dims v_dim .. v_dim + EPL - 1.
+  //
+  // fp32: load c = 4h + j covers dims 64h .. 64h + 63 of tokens 4g + j, g = 0
+  // .. 3: each 16-lane row still reads 256 contiguous bytes of one token, and
+  // lane (grp, row) gets V[token 4grp + j][dims 64h + 4row ..+3], which is
+  // already the A operand of the fp32 P V product (below): V needs no LDS.
   uint32_t kv_off[NL];
   const int v_tok = lane / LPT;
   const int v_dim = EPL * (lane % LPT);
+  auto load_tok = [&](int c) { return FP32 ? 4 * grp + (c & 3) : c * TPL + v_tok; };
+  auto load_dim = [&](int c) { return FP32 ? 64 * (c >> 2) + 4 * row : v_dim; };
 #pragma unroll
   for (int c = 0; c < NL; ++c) {
-    kv_off[c] = static_cast<uint32_t>(((c * TPL + v_tok) * a.token_stride + v_dim) * KB);
+    kv_off[c] = static_cast<uint32_t>((load_tok(c) * a.token_stride + load_dim(c)) * KB);
   }
   // K and V are both loaded row-coalesced (each 16-lane row reads 256
   // contiguous bytes: a token's head dims), which the memory system streams
@@ -542,7 +601,8 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
   // 8 dims), V through the transposing read.
   S* kstage = reinterpret_cast<S*>(lds) + wave * Lds::kWaveStage;
   S* stage = kstage + kBlock * KROW;
-  const S* k_src = kstage + row * KROW + 8 * grp;
+  constexpr int EPC = 16 / E::kBytes;  // elements of a K chunk per lane
+  const S* k_src = kstage + row * KROW + EPC * grp;
   // Source of this lane's 8-byte chunk in the transposing V^T read: token
   // 4grp + row/4, dims 4(row % 4) .. +3 of each 16-wide tile.
   const S* tr_src = stage + (4 * grp + (row >> 2)) * VROW + 4 * (row & 3);
@@ -597,16 +657,15 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
   // no records: the hardware answers with zeros and touches no memory, so no
   // load is still travelling when the waves meet at the merge's barrier
   // (which waits for every outstanding load).
+  auto load_half = [&](const KS* src, u32x4 (&f)[NL], bool live) {
+    const auto r = __builtin_amdgcn_make_buffer_rsrc(const_cast<KS*>(src), static_cast<short>(0),
+                                                     live ? 0x7fffffff : 0, kBufferDword3);
+#pragma unroll
+    for (int c = 0; c < NL; ++c) f[c] = buffer_load16<kKvPolicy>(r, kv_off[c]);
+  };
   auto load_block = [&](int64_t base, u32x4 (&kf)[NL], u32x4 (&vf)[NL], bool live) {
-    const int records = live ? 0x7fffffff : 0;
-    const auto kr = __builtin_amdgcn_make_buffer_rsrc(const_cast<KS*>(kc + base), static_cast<short>(0), records,
-                                                      kBufferDword3);
-    const auto vr = __builtin_amdgcn_make_buffer_rsrc(const_cast<KS*>(vc + base), static_cast<short>(0), records,
-                                                      kBufferDword3);
-#pragma unroll
-    for (int c = 0; c < NL; ++c) kf[c] = buffer_load16<kKvPolicy>(kr, kv_off[c]);
-#pragma unroll
-    for (int c = 0; c < NL; ++c) vf[c] = buffer_load16<kKvPolicy>(vr, kv_off[c]);
+    load_half(kc + base, kf, live);
+    load_half(vc + base, vf, live);
   };
   // One 16-byte load's elements into a staging row as E: a plain store for a
   // 16-bit cache, decoded to two 16-byte chunks for FP8.
@@ -632,13 +691,33 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
 
     // Scores: lane holds S[token 4grp + i][head row] for tile t.
     u32x2 pf[NT], pl[NT];
+    f32x4 p32[NT];  // fp32: the weights as they are
     float alpha[NT];
     bool grew = false;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+      if constexpr (FP32) {
+        // Sums of four products (one MFMA), then a tree over them. One running
+        // sum over all of head_dim rounds more: 16 sequences of up to 4,096
+        // tokens at head_dim 128 were 4.7e-7 off 64 bits with it, 2.3e-7 with
+        // the tree, 3.4e-7 on the VALU kernel.
+        f32x4 part[KC];
 #pragma unroll
-      for (int c = 0; c < KC; ++c) s = M::mma(ka[c], qf[t][c], s);
+        for (int c = 0; c < KC; ++c) {
+          const f32x4 kv = __builtin_bit_cast(f32x4, ka[c]), qv = __builtin_bit_cast(f32x4, qf[t][c]);
+          f32x4 step[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) step[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[j], qv[j], s, 0, 0, 0);
+          part[c] = (step[0] + step[1]) + (step[2] + step[3]);
+#pragma unroll
+          for (int n = 1; ((c + 1) & (2 * n - 1)) == 0; n *= 2) part[c] += part[c - n];
+        }
+        s = part[KC - 1];
+      } else {
+#pragma unroll
+        for (int c = 0; c < KC; ++c) s = M::mma(ka[c], qf[t][c], s);
+      }
       float sc[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) sc[j] = s[j] * qk_scale;
@@ -657,16 +736,24 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
       // normaliser and the log-sum-exp all refer to it. A real block's token
       // 0 is valid, so mx is finite; the first block always moves m off
       // -inf; a padding slot has mx = -inf and leaves m as it is.
-      const float m_new = mx > m[t] + kRescaleSlack ? mx : m[t];
+      const float m_new = mx > m[t] + (FP32 ? 0.0f : kRescaleSlack) ? mx : m[t];
       grew |= m_new > m[t];
       alpha[t] = __builtin_amdgcn_exp2f(m[t] - m_new);
       float p[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) p[j] = __builtin_amdgcn_exp2f(sc[j] - m_new);
+      for (int j = 0; j < 4; ++j) p[j] = __builtin_amdgcn_exp2f(FP32 ? fmaf(s[j], qk_scale, -m_new) : sc[j] - m_new);
+      if (FP32 && nvalid < kBlock) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) p[j] = (4 * grp + j < nvalid) ? p[j] : 0.0f;
+      }
       l[t] = l[t] * alpha[t] + ((p[0] + p[1]) + (p[2] + p[3]));
       m[t] = m_new;
-      pf[t] = u32x2{pack2<E>(p[0], p[1]), pack2<E>(p[2], p[3])};
-      pl[t] = u32x2{pack2_residual<E>(p[0], p[1], pf[t][0]), pack2_residual<E>(p[2], p[3], pf[t][1])};
+      if constexpr (FP32) {
+        p32[t] = f32x4{p[0], p[1], p[2], p[3]};
+      } else {
+        pf[t] = u32x2{pack2<E>(p[0], p[1]), pack2<E>(p[2], p[3])};
+        pl[t] = u32x2{pack2_residual<E>(p[0], p[1], pf[t][0]), pack2_residual<E>(p[2], p[3], pf[t][1])};
+      }
     }
     // Rescale the outputs only when some head's running max moved (alpha < 1).
     if (__any(grew)) {
@@ -680,29 +767,45 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
     stage_v(nvalid);
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
-      const u32x2 va = v_tile(dt);
+      const auto va = v_tile(dt);
 #pragma unroll
-      for (int t = 0; t < NT; ++t) acc[t][dt] = pv_split<E>(va, pf[t], pl[t], acc[t][dt]);
+      for (int t = 0; t < NT; ++t) {
+        if constexpr (FP32) {
+          // k step j: token 4grp + j, whose weight p[j] this lane holds as B.
+          // The block's products are summed on their own, in two halves, so
+          // the long running sum takes one rounding per block.
+          const f32x4 vv = __builtin_bit_cast(f32x4, va);
+          f32x4 step[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const f32x4 before = j < 2 ? f32x4{0.0f, 0.0f, 0.0f, 0.0f} : step[j & 1];
+            step[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[j], p32[t][j], before, 0, 0, 0);
+          }
+          acc[t][dt] += step[2] + step[3];
+        } else {
+          acc[t][dt] = pv_split<E>(va, pf[t], pl[t], acc[t][dt]);
+        }
+      }
     }
   };
 
   // Register pipeline: block i's K and V arrive in registers (kf, vf) and are
   // re-laid out through this wave's LDS tile.
-  auto process_block = [&](int i, const u32x4 (&kf)[NL], const u32x4 (&vf)[NL]) {
+  auto process_block = [&](auto i, const u32x4 (&kf)[NL], const u32x4 (&vf)[NL]) {
     // Stage K (its rows past seq_len only feed scores replaced by -inf).
 #pragma unroll
-    for (int c = 0; c < NL; ++c) stage16(kstage + (c * TPL + v_tok) * KROW + v_dim, kf[c]);
+    for (int c = 0; c < NL; ++c) stage16(kstage + load_tok(c) * KROW + load_dim(c), kf[c]);
     u32x4 ka[KC];
 #pragma unroll
-    for (int c = 0; c < KC; ++c) ka[c] = *reinterpret_cast<const u32x4*>(k_src + 32 * c);
+    for (int c = 0; c < KC; ++c) ka[c] = *reinterpret_cast<const u32x4*>(k_src + 4 * EPC * c);
     compute_block(
         i, ka,
         [&](int nvalid) {
           // Stage V, rows past seq_len as zeros, for the transposed reads.
 #pragma unroll
           for (int c = 0; c < NL; ++c) {
-            const int tok = c * TPL + v_tok;
-            stage16(stage + tok * VROW + v_dim, tok < nvalid ? vf[c] : u32x4{0, 0, 0, 0});
+            const int tok = load_tok(c);
+            stage16(stage + tok * VROW + load_dim(c), tok < nvalid ? vf[c] : u32x4{0, 0, 0, 0});
           }
         },
         [&](int dt) { return lds_read_tr16(tr_src + 16 * dt); });
@@ -777,6 +880,46 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
       // loads in flight into LDS that the cross-wave merge reuses.
       wait_vmcnt<0>();
     }
+  } else if constexpr (FP32) {
+    // fp32: a block is 64 registers per lane and two of them leave one wave per
+    // SIMD, so K and V take turns in one block's registers. K moves on to LDS
+    // before it is used and V is used last: block i + 1's K is loaded once
+    // block i's is staged and travels while block i is computed, its V follows
+    // block i's P V product and travels through block i + 1's scores. The
+    // block-table entry of block i + 2 is loaded ahead of both, so its wait
+    // leaves them in flight (vector loads complete in order).
+    u32x4 kf[NL], vf[NL];
+    if (nblk > 0) {
+      float pg = page_load(min(1, nblk - 1));
+      const int64_t base0 = block_base(0);
+      load_block(base0, kf, vf, true);
+      for (int i = 0; i < nblk; ++i) {
+        const bool more = i + 1 < nblk;
+        const int64_t next = page_base(min(i + 1, nblk - 1), __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, pg)));
+        pg = page_load(min(i + 2, nblk - 1));
+#pragma unroll
+        for (int c = 0; c < NL; ++c) stage16(kstage + load_tok(c) * KROW + load_dim(c), kf[c]);
+        load_half(kc + next, kf, more);
+        u32x4 ka[KC];
+#pragma unroll
+        for (int c = 0; c < KC; ++c) ka[c] = *reinterpret_cast<const u32x4*>(k_src + 4 * EPC * c);
+        compute_block(
+            i, ka,
+            [&](int nvalid) {
+              // Rows past seq_len count as zeros.
+              if (nvalid < kBlock) {
+#pragma unroll
+                for (int c = 0; c < NL; ++c) vf[c] = load_tok(c) < nvalid ? vf[c] : u32x4{0, 0, 0, 0};
+              }
+            },
+            // Tile dt = 4h + e: element e of the four loads of dims 64h ..
+            [&](int dt) {
+              const int h = dt & ~3, e = dt & 3;
+              return u32x4{vf[h][e], vf[h + 1][e], vf[h + 2][e], vf[h + 3][e]};
+            });
+        load_half(vc + next, vf, more);
+      }
+    }
   } else if (nblk > 0) {
     // NS-stage pipeline: while block i is processed, blocks i+1 .. i+NS-1 are
     // in flight. The loop runs a whole number of NS-block rounds with no
@@ -838,10 +981,18 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
       lds_ml[((wave * NT + t) * 16 + lane) * 2 + 1] = l[t];
     }
   }
+  // Chunk dt holds four consecutive output dims per lane: the tile itself, dims
+  // 16dt + 4grp ..+3, in 16 bits; in fp32, whose tile 4h + e is the dims 64h +
+  // 4r + e (r: the tile's row, 4grp + i), element i of tiles 4h .. 4h + 3, dims
+  // 64h + 16grp + 4i ..+3.
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) lds_acc[(wave * NT * DT + t * DT + dt) * 64 + lane] = acc[t][dt];
+    for (int dt = 0; dt < DT; ++dt) {
+      const int h = dt & ~3, i = dt & 3;
+      lds_acc[(wave * NT * DT + t * DT + dt) * 64 + lane] =
+          FP32 ? f32x4{acc[t][h][i], acc[t][h + 1][i], acc[t][h + 2][i], acc[t][h + 3][i]} : acc[t][dt];
+    }
   }
   __syncthreads();
 
@@ -876,12 +1027,16 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
       for (int w = 1; w < W; ++w) num += lds_acc[(w * NT * DT + t * DT + dt) * 64 + lane] * cw[w];
       float o[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] = num[i] * inv;
+      for (int i = 0; i < 4; ++i) o[i] = FP32 ? num[i] / denom : num[i] * inv;
       if (!valid) continue;
-      const int d = 16 * dt + 4 * grp;
+      const int d = FP32 ? 16 * (dt & ~3) + 16 * grp + 4 * (dt & 3) : 16 * dt + 4 * grp;
       if (dst.final) {
         S* out = static_cast<S*>(a.out) + head * D + d;
-        *reinterpret_cast<u32x2*>(out) = u32x2{pack2<E>(o[0], o[1]), pack2<E>(o[2], o[3])};
+        if constexpr (FP32) {
+          *reinterpret_cast<f32x4*>(out) = f32x4{o[0], o[1], o[2], o[3]};
+        } else {
+          *reinterpret_cast<u32x2*>(out) = u32x2{pack2<E>(o[0], o[1]), pack2<E>(o[2], o[3])};
+        }
       } else {
         // Partials are stored device-coherent: with the fused merge, a
         // workgroup on another XCD reads them within this launch.
@@ -1079,8 +1234,11 @@ __device__ __forceinline__ Dest uniform_dest(const DecodeArgs& a, const Unit& u,
 // Uniform splits: workgroup = (sequence, KV head, head group, split), the
 // split owning pages_per_split pages (the reference's decomposition).
 template <typename E, typename KVF, int D, int NT>
-__global__ void __launch_bounds__(kThreads, (mfma_waves_per_eu<D, NT>())) decode_mfma_kernel(const DecodeArgs a) {
-  __shared__ __attribute__((aligned(16))) char lds[MfmaLds<D, NT, kWaves, dma_staged<KVF, D, NT>()>::kBytes];
+__global__ void __launch_bounds__((uniform_waves<E, D, NT>() * 64), (mfma_waves_per_eu<D, NT, E>()))
+    decode_mfma_kernel(const DecodeArgs a) {
+  constexpr int W = uniform_waves<E, D, NT>();
+  __shared__ __attribute__((
+      aligned(16))) char lds[MfmaLds<D, NT, W, dma_staged<KVF, D, NT>(), kDmaStages, E::kBytes>::kBytes];
   __shared__ int s_last[1];
   fetch_args(a);
   // q and the first block-table window depend on the unit alone: they are
@@ -1088,10 +1246,10 @@ __global__ void __launch_bounds__(kThreads, (mfma_waves_per_eu<D, NT>())) decode
   // follow one memory round trip after it instead of two.
   Unit u = decode_unit_ids(a);
   const int wave = wave_id();
-  QFrag<NT, D / 32> q;
+  QFrag<NT, qk_chunks<E, D>()> q;
   load_q<E, D, NT>(a, u, q);
   const int pb = u.split * a.pages_per_split;
-  prefetch_window<KVF, D, NT>(a, lds, u.b, pb, min(pb + a.pages_per_split, a.max_pages), wave);
+  prefetch_window<KVF, D, NT, W>(a, lds, u.b, pb, min(pb + a.pages_per_split, a.max_pages), wave);
   unit_pages(a, u);
   if (u.page_begin >= u.page_end) {
     wait_vmcnt<0>();  // the window loads write this workgroup's LDS
@@ -1101,10 +1259,10 @@ __global__ void __launch_bounds__(kThreads, (mfma_waves_per_eu<D, NT>())) decode
     return;  // a split past the end of its sequence has no work
   }
   const Dest dst = uniform_dest(a, u, D);
-  mfma_segment<E, KVF, D, NT>(a, lds, u, dst, wave, &q, true);
+  mfma_segment<E, KVF, D, NT, W>(a, lds, u, dst, wave, &q, true);
   if constexpr (NT == 1) {  // see kFusedMergeMaxHeads
     if (!dst.final && a.arrivals != nullptr) {
-      arrive_and_merge<E>(unit_counter(a, u), uniform_job<E>(a, u, D, active_splits(a, u)), D, wave_id(), s_last);
+      arrive_and_merge<E, W>(unit_counter(a, u), uniform_job<E>(a, u, D, active_splits(a, u)), D, wave_id(), s_last);
     }
   }
 }
@@ -1133,7 +1291,7 @@ __global__ void __launch_bounds__(2 * kThreads, (mfma_waves_per_eu<D, NT>()))
   fetch_args(a);
   // q and the first block-table window before seq_lens (decode_mfma_kernel).
   Unit u = decode_unit_paired_ids(a, half);
-  QFrag<NT, D / 32> q;
+  QFrag<NT, qk_chunks<E, D>()> q;
   load_q<E, D, NT>(a, u, q);
   const int pb = u.split * a.pages_per_split;
   prefetch_window<KVF, D, NT>(a, lds + half * Lds::kBytes, u.b, pb, min(pb + a.pages_per_split, a.max_pages),
@@ -1484,7 +1642,7 @@ __global__ void __launch_bounds__(PAIR * kThreads, (mfma_waves_per_eu<D, NT>()))
   // the main loops compiled to the same instructions; q after the window
   // and seq_lens costs nothing measurable.
   Unit gu{};
-  QFrag<NT, D / 32> gq;
+  QFrag<NT, qk_chunks<E, D>()> gq;
   if (a.even_start) {
     gu = list_unit<PAIR>(a, hp, w, half);
     prefetch_window<KVF, D, NT>(a, lds + half * Lds::kBytes, gu.b, 0, a.max_pages, hw);
@@ -2110,8 +2268,10 @@ void set_page_size(DecodeArgs& a, int page_size) {
 
 // Shapes the MFMA kernels serve.
 bool mfma_path(kl_dtype dtype, int head_dim, int page_size) {
-  return (dtype == KL_DTYPE_F16 || dtype == KL_DTYPE_BF16) && page_size % kBlock == 0 &&
-         (head_dim == 32 || head_dim == 64 || head_dim == 128 || head_dim == 256);
+  if (page_size % kBlock != 0) return false;
+  if (head_dim == 64 || head_dim == 128 || head_dim == 256) return true;
+  // fp32's V operand takes 64 head dims at a time.
+  return head_dim == 32 && dtype != KL_DTYPE_F32;
 }
 
 // Switches for A/B measurements and tests; unset, the library behaves as
@@ -2362,6 +2522,7 @@ int make_plan(const Options& opt, kl_dtype dtype, int batch, int num_q_heads, in
     return fail(KL_ERR_UNSUPPORTED, "dtype must be f32, f16 or bf16");
   }
   const bool mfma = use_mfma && mfma_path(dtype, head_dim, page_size);
+  const bool mfma16 = mfma && dtype != KL_DTYPE_F32;  // fp32 runs uniform splits, one KV head per workgroup
   if (!mfma && !valu_head_dim_ok(dtype, head_dim)) {
     return fail(KL_ERR_UNSUPPORTED, "head_dim must be 16, 32, 64, 128 or 256");
   }
@@ -2372,7 +2533,7 @@ int make_plan(const Options& opt, kl_dtype dtype, int batch, int num_q_heads, in
   p->paired = false;
   const int cus = cu_count > 0 ? cu_count : 256;
   const int64_t units = std::max<int64_t>(1, static_cast<int64_t>(batch) * num_kv_heads * p->head_groups);
-  if (num_splits == KL_SPLITS_BALANCED && (!mfma || partials)) num_splits = 0;  // uniform splits only
+  if (num_splits == KL_SPLITS_BALANCED && (!mfma16 || partials)) num_splits = 0;  // uniform splits only
   // The balanced schedule runs in KV-head pairs (8-wave workgroups) on
   // batches that fill the device twice over, as uniform splits would, and on
   // long contexts that give every workgroup half long segments of few-way
@@ -2380,7 +2541,7 @@ int make_plan(const Options& opt, kl_dtype dtype, int batch, int num_q_heads, in
   const int64_t pair_units = units / 2;
   const bool long_pairs = pair_units * pages >= static_cast<int64_t>(cus) * kPairMinPages &&
                           pair_units * kPairMaxSegments >= cus;
-  const bool pairable = mfma && !partials && opt.pairing() && num_kv_heads % 2 == 0 && head_dim <= 128 &&
+  const bool pairable = mfma16 && !partials && opt.pairing() && num_kv_heads % 2 == 0 && head_dim <= 128 &&
                         p->heads_per_wg <= 16 && (units >= 2 * static_cast<int64_t>(cus) || long_pairs);
   // Batches whose units fill the device (units >= CUs) take the balanced
   // schedule too. The planner cannot see seq_lens, and with uniform splits
@@ -2418,7 +2579,7 @@ int make_plan(const Options& opt, kl_dtype dtype, int batch, int num_q_heads, in
       (units < cus || (full_batch_choice < 0 ? full_default : full_batch_choice == 1));
   const bool balance = requested || automatic;
   const bool pair_balanced = pairable && balance;
-  if (mfma && !partials && balance) {
+  if (mfma16 && !partials && balance) {
     // Requested, fewer units than CUs, or a full batch by default: pages
     // balanced across sequences on the device.
     const int64_t lunits = pair_balanced ? units / 2 : units;  // units of the work list
@@ -2495,7 +2656,7 @@ int make_plan(const Options& opt, kl_dtype dtype, int batch, int num_q_heads, in
   // Two adjacent KV heads per 8-wave workgroup when the pairs alone give
   // every CU a workgroup (one 8-wave workgroup per CU is the register budget)
   // and the 4-wave kernel fits two waves per SIMD (head_dim <= 128).
-  p->paired = mfma && opt.pairing() && num_kv_heads % 2 == 0 && head_dim <= 128 && units * s / 2 >= cus;
+  p->paired = mfma16 && opt.pairing() && num_kv_heads % 2 == 0 && head_dim <= 128 && units * s / 2 >= cus;
   if (s > 1 || partials) {
     const size_t rows = static_cast<size_t>(batch) * num_q_heads * s;
     p->o_bytes = align_up(rows * head_dim * sizeof(float));
@@ -2563,7 +2724,7 @@ int dispatch_mfma(int head_dim, int heads_per_wg, F&& f) {
 // head_dim >= 64.
 template <typename KVF, int D>
 constexpr bool mfma_instance_exists() {
-  return KVF::kBytes == 2 || D >= 64;
+  return KVF::kBytes == 2 || D >= 64;  // fp32 too: see mfma_path
 }
 
 template <typename E>
@@ -2609,15 +2770,15 @@ int launch_uniform_mfma(const DecodeArgs& a, int head_dim, unsigned grid, hipStr
     constexpr int D = decltype(d)::value, NT = decltype(nt)::value;
     if constexpr (mfma_instance_exists<KVF, D>()) {
       if (a.paired) {
-        // head_dim 256 is never paired: its segment needs more than the
-        // 256 registers per lane an 8-wave workgroup leaves.
-        if constexpr (D <= 128) {
+        // head_dim 256 and fp32 are never paired: the segment needs more than
+        // the 256 registers per lane an 8-wave workgroup leaves.
+        if constexpr (D <= 128 && !std::is_same_v<E, F32>) {
           decode_mfma_paired_kernel<E, KVF, D, NT><<<grid / 2, 2 * kThreads, 0, stream>>>(a);
         } else {
-          return fail(KL_ERR_UNSUPPORTED, "paired decode needs head_dim <= 128");
+          return fail(KL_ERR_UNSUPPORTED, "paired decode needs 16-bit queries and head_dim <= 128");
         }
       } else {
-        decode_mfma_kernel<E, KVF, D, NT><<<grid, kThreads, 0, stream>>>(a);
+        decode_mfma_kernel<E, KVF, D, NT><<<grid, uniform_waves<E, D, NT>() * 64, 0, stream>>>(a);
       }
       return KL_OK;
     } else {
@@ -2682,7 +2843,7 @@ int launch_balanced(DecodeArgs a, int head_dim, hipStream_t stream) {
 template <typename E, typename KVF>
 int launch_typed(DecodeArgs& a, int head_dim, bool mfma, hipStream_t stream) {
   if constexpr (std::is_same_v<E, F32>) {
-    if (mfma || a.grid > 0) return fail(KL_ERR_UNSUPPORTED, "fp32 runs on the VALU path only");
+    if (a.grid > 0) return fail(KL_ERR_UNSUPPORTED, "fp32 has no balanced schedule");
   }
   if (a.grid > 0) {
     if constexpr (!std::is_same_v<E, F32>) return launch_balanced<E, KVF>(a, head_dim, stream);
@@ -2692,13 +2853,8 @@ int launch_typed(DecodeArgs& a, int head_dim, bool mfma, hipStream_t stream) {
   if (mfma && a.num_splits > 1) {
     a.arrivals = fused_merge_counters(a, static_cast<int64_t>(a.batch) * a.num_kv_heads * a.head_groups, stream);
   }
-  int st;
-  if constexpr (!std::is_same_v<E, F32>) {
-    st = mfma ? launch_uniform_mfma<E, KVF>(a, head_dim, static_cast<unsigned>(wgs), stream)
-              : launch_valu<E>(a, head_dim, static_cast<unsigned>(wgs), stream);
-  } else {
-    st = launch_valu<E>(a, head_dim, static_cast<unsigned>(wgs), stream);
-  }
+  int st = mfma ? launch_uniform_mfma<E, KVF>(a, head_dim, static_cast<unsigned>(wgs), stream)
+                : launch_valu<E>(a, head_dim, static_cast<unsigned>(wgs), stream);
   if (st != KL_OK) return st;
   st = check_launch("paged decode split kernel launch");
   if (st != KL_OK) return st;
@@ -2814,7 +2970,7 @@ int decode_entry(kl_dtype dtype, bool kv8, void* out, const void* q, const void*
   const bool mfma = use_mfma && mfma_path(dtype, head_dim, page_size);
   switch (dtype) {
     case KL_DTYPE_F32:
-      return launch_typed<F32, F32>(a, head_dim, false, stream);
+      return launch_typed<F32, F32>(a, head_dim, mfma, stream);
     case KL_DTYPE_F16:
       return kv8 ? launch_typed<F16, Fp8E4M3>(a, head_dim, true, stream)
                  : launch_typed<F16, F16>(a, head_dim, mfma, stream);

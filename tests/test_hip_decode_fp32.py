@@ -1,0 +1,47 @@
+"""fp32 decode on the matrix cores, at the sizes where it can go wrong.
+
+Lengths end inside, on and just past a 16-token block, a round of the
+workgroup's waves (8 waves x 16 tokens; 4 x 16 where it runs four) and a page;
+tails and spare pages hold NaN. Groups fill one head tile partly, wholly, and
+two tiles (17 to 32 query heads per KV head) or several head groups. The oracle
+is the float32 CPU path; decode_parity allows one fp32 ulp plus 1e-6.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from kernel_lab.kv_cache import random_decode_problem
+from oracle import reference as ref
+from tests.conftest import decode_parity
+
+pytestmark = pytest.mark.gpu
+
+LENS = [1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 255, 257, 700]
+
+
+@pytest.mark.parametrize("head_dim", [64, 128, 256])
+@pytest.mark.parametrize(("hq", "hkv"), [(3, 3), (8, 2), (16, 1), (20, 1), (32, 1), (80, 2)])
+@pytest.mark.parametrize("splits", [None, 1, 3])
+def test_fp32_mfma_edges(gpu_ops, head_dim, hq, hkv, splits):
+    page = 48 if splits == 3 else 16
+    q, kv, _, _ = random_decode_problem(LENS, hq, hkv, head_dim, page, dtype=torch.float32, device="cuda",
+                                        poison=float("nan"), tail=float("nan"), seed=head_dim + hq)
+    out = gpu_ops.paged_decode_attention(q, kv.k_cache, kv.v_cache, kv.block_table, kv.seq_lens, num_splits=splits)
+    want = ref.paged_decode_attention(q.cpu(), kv.k_cache.cpu(), kv.v_cache.cpu(), kv.block_table.cpu(), kv.seq_lens.cpu())
+    decode_parity(out, want, torch.float32, f"{hq}/{hkv}/{head_dim} splits {splits}")
+
+
+@pytest.mark.parametrize("head_dim", [64, 128, 256])
+def test_fp32_mfma_is_no_further_from_64_bits_than_torch(gpu_ops, head_dim):
+    """The scores and the block sums are added as trees: the result stays
+    within 4e-7 (about three fp32 roundings in the 2-norm) of 64 bits."""
+    q, kv, keys, values = random_decode_problem([2000, 333], 8, 2, head_dim, 16, dtype=torch.float32, device="cuda")
+    out = gpu_ops.paged_decode_attention(q, kv.k_cache, kv.v_cache, kv.block_table, kv.seq_lens).cpu().double()
+    for b in range(2):
+        k = keys[b].cpu().double().transpose(0, 1)
+        v = values[b].cpu().double().transpose(0, 1)
+        w = torch.softmax(q[b].cpu().double().reshape(2, 4, head_dim) @ k.transpose(1, 2) * head_dim**-0.5, -1)
+        want = (w @ v).reshape(8, head_dim)
+        assert (out[b] - want).norm() <= 4e-7 * want.norm()
