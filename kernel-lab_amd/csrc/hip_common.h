@@ -12,6 +12,7 @@
 #include <stdint.h>
 
 #include <type_traits>
+#include <utility>
 
 namespace kl {
 
@@ -133,6 +134,22 @@ template <int CTRL>
 __device__ __forceinline__ float dpp(float v) {
   return __builtin_bit_cast(
       float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+}
+
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
+  return static_cast<uint32_t>(
+      __builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, 0xF, 0xF, false));
+}
+
+// f(std::integral_constant<int, 0>) .. f(std::integral_constant<int, N - 1>).
+template <int N, typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl<N>(f, std::make_integer_sequence<int, N>{});
 }
 
 __device__ __forceinline__ float lane_read(float v, int lane) {
@@ -273,6 +290,12 @@ __device__ __forceinline__ void buffer_store16(__amdgpu_buffer_rsrc_t rsrc, uint
 template <int POLICY = 0>
 __device__ __forceinline__ void buffer_store_f32(__amdgpu_buffer_rsrc_t rsrc, uint32_t byte_offset, float v) {
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rsrc, byte_offset, 0, POLICY);
+}
+
+// Non-temporal 16-byte load from a 64-bit per-lane address.
+__device__ __forceinline__ u32x4 global_load16_nt(const char* p) {
+  typedef const __attribute__((address_space(1))) u32x4* global_u32x4;
+  return __builtin_nontemporal_load((global_u32x4)(p));
 }
 
 // Waits until every vector memory access this wave issued has completed

@@ -24,7 +24,8 @@
 // log2-sum-exp, and a merge kernel combines the partials of each (sequence,
 // query head).
 //
-// MFMA path (fp16 / bf16, page_size % 16 == 0, head_dim in {32,64,128,256}):
+// MFMA path (fp16 / bf16, head_dim in {32,64,128,256}; pages that do not hold
+// whole 16-token blocks: see SmallPages):
 //   S  = K . Q^T    v_mfma_f32_16x16x32_{f16,bf16}: rows = 16 tokens of a
 //                   block, columns = up to 16 query heads of the GQA group.
 //                   K is loaded row-coalesced (16 lanes read one token's head
@@ -43,7 +44,7 @@
 // garbage there cannot leak; pages past cdiv(seq_len, page_size) and pages not
 // named by the block table are never read.
 //
-// MFMA path in fp32 (page_size % 16 == 0, head_dim in {64,128,256}): the same
+// MFMA path in fp32 (head_dim in {64,128,256}): the same
 // segment on v_mfma_f32_16x16x4_f32, operands, weights and sums in fp32.
 //   S = K . Q^T     K restaged through LDS as above; a lane's 16 bytes are four
 //                   k steps.
@@ -139,6 +140,13 @@ struct DecodeArgs {
   uint32_t bpp_magic;
   int bpp_shift;
   int max_pages;
+  int max_len;          // longest length a sequence may have: seq_lens beyond it count as it
+  // Caches whose pages do not hold whole blocks (SmallPages): the block table's
+  // page size, and the division by it. page_size and max_pages are then the
+  // schedule's, which need not be the table's.
+  int table_page;
+  uint32_t table_magic;
+  int table_shift;
   int num_splits;
   int pages_per_split;
   int head_groups;      // workgroups per (sequence, KV head, split) along the group
@@ -172,6 +180,25 @@ __device__ __forceinline__ int block_page(const DecodeArgs& a, int n) {
   return static_cast<int>((static_cast<uint64_t>(static_cast<uint32_t>(n)) * a.bpp_magic) >> a.bpp_shift);
 }
 
+// Token index -> column of the block table, for a SmallPages cache.
+__device__ __forceinline__ int table_column(const DecodeArgs& a, int tok) {
+  return static_cast<int>((static_cast<uint64_t>(static_cast<uint32_t>(tok)) * a.table_magic) >> a.table_shift);
+}
+
+// Cache format F on pages that do not hold whole 16-token blocks (page_size not
+// a multiple of 16), so a block's tokens come from several pages: every lane
+// addresses its own token's row instead of the wave one block. The rows stay
+// whole and coalesced, so HBM and the segment starts bound it as they do the
+// other caches; the addresses cost about 40 VALU instructions a block. Measured
+// (us, VALU kernel -> this): 32/8/128 bf16 page 8 B=32 up to 2,048 tokens 207 ->
+// 30.5.
+template <typename F>
+struct SmallPages : F {};
+template <typename KVF>
+constexpr bool kSmallPages = false;
+template <typename F>
+constexpr bool kSmallPages<SmallPages<F>> = true;
+
 struct Unit {
   int b, kvh, hg, split;
   int seq_len;          // clamped to max_pages * page_size
@@ -182,8 +209,7 @@ struct Unit {
 // split are set.
 __device__ __forceinline__ void unit_pages(const DecodeArgs& a, Unit& u) {
   const int raw = as_constant(a.seq_lens)[u.b];
-  const int64_t cap = static_cast<int64_t>(a.max_pages) * a.page_size;
-  u.seq_len = static_cast<int>(raw < cap ? raw : cap);
+  u.seq_len = min(raw, a.max_len);
   const int num_pages = u.seq_len > 0 ? (u.seq_len + a.page_size - 1) / a.page_size : 0;
   u.page_begin = u.split * a.pages_per_split;
   u.page_end = min(u.page_begin + a.pages_per_split, num_pages);
@@ -351,7 +377,7 @@ struct MfmaLds {
 // those keep registers.
 template <typename KVF, int D, int NT>
 constexpr bool dma_staged() {
-  return KVF::kBytes == 2 && D == 128 && NT == 1;
+  return KVF::kBytes == 2 && !kSmallPages<KVF> && D == 128 && NT == 1;
 }
 
 // Register pipeline depth: blocks whose K and V are held in VGPRs at once
@@ -408,12 +434,15 @@ struct Dest {
 // such load in turn; the uniform decode kernel's prologue showed three
 // dependent argument round trips before its first q load. Naming the fields
 // the kernels read as inputs of an empty asm statement has them loaded before
-// it, with one wait.
+// it, with one wait. kWindow: the kernel loads block-table windows, the only
+// readers of max_pages.
+template <bool kWindow>
 __device__ __forceinline__ void fetch_args(const DecodeArgs& a) {
+  if constexpr (kWindow) asm volatile("" ::"s"(a.max_pages));
   asm volatile("" ::"s"(a.q), "s"(a.k), "s"(a.v), "s"(a.out), "s"(a.block_table), "s"(a.seq_lens), "s"(a.o_part),
                "s"(a.lse_part), "s"(a.bt_stride), "s"(a.page_stride), "s"(a.arrivals));
   asm volatile("" ::"s"(a.token_stride), "s"(a.batch), "s"(a.num_q_heads), "s"(a.num_kv_heads), "s"(a.group),
-               "s"(a.page_size), "s"(a.bpp_magic), "s"(a.bpp_shift), "s"(a.max_pages), "s"(a.num_splits),
+               "s"(a.page_size), "s"(a.bpp_magic), "s"(a.bpp_shift), "s"(a.max_len), "s"(a.num_splits),
                "s"(a.pages_per_split), "s"(a.head_groups), "s"(a.heads_per_wg), "s"(a.grid), "s"(a.even_start),
                "s"(a.seg_charge), "s"(a.scale_log2),
                "s"(a.q_fold), "s"(a.q_heads), "s"(a.force_partial));
@@ -513,6 +542,7 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
   using M = Mfma<E>;
   constexpr bool KV8 = std::is_same_v<KVF, Fp8E4M3>;
   constexpr bool FP32 = std::is_same_v<E, F32>;
+  constexpr bool SP = kSmallPages<KVF>;
   constexpr int KB = KVF::kBytes;      // cache bytes per element
   constexpr int KC = qk_chunks<E, D>();  // QK k-chunks
   constexpr int DT = D / 16;           // PV output tiles along head_dim
@@ -570,11 +600,22 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
   }
   const const_i32_ptr bt = as_constant(a.block_table + static_cast<int64_t>(u.b) * a.bt_stride);
   const int bpp = a.page_size / kBlock;  // blocks per page
-  const int blk_begin = u.page_begin * bpp;
-  const int blk_end = min(u.page_end * bpp, (u.seq_len + kBlock - 1) / kBlock);
+  const int blk_begin = SP ? 0 : u.page_begin * bpp;
+  // Small pages: the segment's tokens tok0 .. tok_end - 1, its blocks counted from tok0.
+  const int tok0 = u.page_begin * a.page_size;
+  const int tok_end =
+      static_cast<int>(min(static_cast<int64_t>(u.page_end) * a.page_size, static_cast<int64_t>(u.seq_len)));
+  const int blk_end = SP ? (tok_end - tok0 + kBlock - 1) / kBlock
+                         : min(u.page_end * bpp, (u.seq_len + kBlock - 1) / kBlock);
   // This wave's blocks: blk_begin + wave + W * i, i < nblk.
   const int first = blk_begin + wave;
   const int nblk = first < blk_end ? (blk_end - first + W - 1) / W : 0;
+  // Valid tokens of block i: >= 16 means all; <= 0 only for the padding slots
+  // of the last pipeline round (i >= nblk).
+  auto valid_of = [&](int i) {
+    if constexpr (SP) return i < nblk ? tok_end - tok0 - (first + W * i) * kBlock : 0;
+    return i < nblk ? u.seq_len - (first + W * i) * kBlock : 0;
+  };
 
   // Per-lane byte offsets inside a block (token row x head dims), for buffer
   // loads off a per-block wave-uniform base. Load c covers tokens
@@ -588,7 +629,8 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
   uint32_t kv_off[NL];
   const int v_tok = lane / LPT;
   const int v_dim = EPL * (lane % LPT);
-  auto load_tok = [&](int c) { return FP32 ? 4 * grp + (c & 3) : c * TPL + v_tok; };
+  // Small pages, 16 bits: NL consecutive tokens per LPT lanes (block_src).
+  auto load_tok = [&](int c) { return FP32 ? 4 * grp + (c & 3) : SP ? NL * v_tok + c : c * TPL + v_tok; };
   auto load_dim = [&](int c) { return FP32 ? 64 * (c >> 2) + 4 * row : v_dim; };
 #pragma unroll
   for (int c = 0; c < NL; ++c) {
@@ -652,20 +694,99 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
   auto page_load = [&](int i) -> float {
     return buffer_load_f32(btr, static_cast<uint32_t>(block_page(a, first + W * i)) * 4u);
   };
+  // Small pages: the tokens a lane loads (load_tok) are the same for the four
+  // lanes of a quad, so lane c of the quad looks up token c (and c + 4, where a
+  // lane loads eight): one table entry and one address each instead of one per
+  // load, passed round the quad by DPP when the loads go out. Tokens past the
+  // segment take its last one's row, which is read again and masked later.
+  constexpr int NTOK = FP32 ? 4 : NL;             // distinct tokens a lane loads
+  constexpr int NE = NTOK > 4 ? NTOK / 4 : 1;     // table entries per lane
+  struct Entries {
+    float e[NE];
+  };
+  struct Rows {
+    uint32_t lo[NE], hi[NE];  // byte offset of the token's row in the cache
+  };
+  auto own_tok = [&](int i, int n) {
+    const int c = 4 * n + (lane & (NTOK < 4 ? NTOK - 1 : 3));
+    return min(tok0 + (first + W * i) * kBlock + load_tok(c), tok_end - 1);
+  };
+  auto entries_load = [&](int i) {
+    Entries r;
+#pragma unroll
+    for (int n = 0; n < NE; ++n) {
+      r.e[n] = buffer_load_f32(btr, static_cast<uint32_t>(table_column(a, own_tok(i, n))) * 4u);
+    }
+    return r;
+  };
+  auto block_rows = [&](int i, const Entries& en) {
+    Rows r;
+#pragma unroll
+    for (int n = 0; n < NE; ++n) {
+      const int tok = own_tok(i, n);
+      const int slot = tok - table_column(a, tok) * a.table_page;
+      const uint64_t row = static_cast<uint64_t>(__builtin_bit_cast(uint32_t, en.e[n])) *
+                               static_cast<uint32_t>(a.table_page) + static_cast<uint32_t>(slot);
+      const uint64_t off = row * static_cast<uint32_t>(a.token_stride * KB);
+      r.lo[n] = static_cast<uint32_t>(off);
+      r.hi[n] = static_cast<uint32_t>(off >> 32);
+    }
+    return r;
+  };
+  auto load_rows = [&](const KS* cache, const Rows& r, u32x4 (&f)[NL]) {
+    static_for<NL>([&](auto cc) {
+      constexpr int c = decltype(cc)::value;
+      constexpr int n = FP32 ? 0 : c / 4;
+      constexpr int kFromLane = (c & 3) * 0x55;  // quad_perm [c,c,c,c]
+      const uint32_t lo = NTOK == 1 ? r.lo[n] : dpp_u32<kFromLane>(r.lo[n]);
+      const uint32_t hi = NTOK == 1 ? r.hi[n] : dpp_u32<kFromLane>(r.hi[n]);
+      const uint64_t off = (static_cast<uint64_t>(hi) << 32) | lo;
+      f[c] = global_load16_nt(reinterpret_cast<const char*>(cache + static_cast<int64_t>(u.kvh) * D + load_dim(c)) + off);
+    });
+  };
 
   // A padding slot of the last round (live false) loads through resources of
   // no records: the hardware answers with zeros and touches no memory, so no
   // load is still travelling when the waves meet at the merge's barrier
   // (which waits for every outstanding load).
-  auto load_half = [&](const KS* src, u32x4 (&f)[NL], bool live) {
-    const auto r = __builtin_amdgcn_make_buffer_rsrc(const_cast<KS*>(src), static_cast<short>(0),
-                                                     live ? 0x7fffffff : 0, kBufferDword3);
-#pragma unroll
-    for (int c = 0; c < NL; ++c) f[c] = buffer_load16<kKvPolicy>(r, kv_off[c]);
+  //
+  // table_load, block_src, first_src and load_half stand for either addressing:
+  // a block's table entry (or the lane's entries), its source from that entry,
+  // a first block's source outright, and one cache's loads from a source.
+  auto table_load = [&](int i) {
+    if constexpr (SP) {
+      return entries_load(i);
+    } else {
+      return page_load(i);
+    }
   };
-  auto load_block = [&](int64_t base, u32x4 (&kf)[NL], u32x4 (&vf)[NL], bool live) {
-    load_half(kc + base, kf, live);
-    load_half(vc + base, vf, live);
+  auto block_src = [&](int i, const auto& entry) {
+    if constexpr (SP) {
+      return block_rows(i, entry);
+    } else {
+      return page_base(i, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, entry)));
+    }
+  };
+  auto first_src = [&](int i) {
+    if constexpr (SP) {
+      return block_rows(i, entries_load(i));
+    } else {
+      return block_base(i);
+    }
+  };
+  auto load_half = [&](const KS* cache, const auto& src, u32x4 (&f)[NL], bool live) {
+    if constexpr (SP) {
+      load_rows(cache, src, f);
+    } else {
+      const auto r = __builtin_amdgcn_make_buffer_rsrc(const_cast<KS*>(cache + src), static_cast<short>(0),
+                                                       live ? 0x7fffffff : 0, kBufferDword3);
+#pragma unroll
+      for (int c = 0; c < NL; ++c) f[c] = buffer_load16<kKvPolicy>(r, kv_off[c]);
+    }
+  };
+  auto load_block = [&](const auto& src, u32x4 (&kf)[NL], u32x4 (&vf)[NL], bool live) {
+    load_half(kc, src, kf, live);
+    load_half(vc, src, vf, live);
   };
   // One 16-byte load's elements into a staging row as E: a plain store for a
   // 16-bit cache, decoded to two 16-byte chunks for FP8.
@@ -685,9 +806,7 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
   // a stage_v(nvalid) step run before the V tiles are read, and v_tile(dt),
   // which reads V^T tile dt (lane holds V[token 4grp + j][dim 16dt + row]).
   auto compute_block = [&](int i, const u32x4 (&ka)[KC], auto&& stage_v, auto&& v_tile) {
-    // Valid tokens in the block: >= 16 means all; <= 0 only for the padding
-    // slots of the last pipeline round (i >= nblk).
-    const int nvalid = i < nblk ? u.seq_len - (first + W * i) * kBlock : 0;
+    const int nvalid = valid_of(i);
 
     // Scores: lane holds S[token 4grp + i][head row] for tile t.
     u32x2 pf[NT], pl[NT];
@@ -860,7 +979,6 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
 #pragma unroll
         for (int c = 0; c < NL; ++c) buffer_load16_lds_nt(vc + off, records, dst + kBlock * D * 2 + c * 1024, v_off[c]);
       };
-      auto valid_of = [&](int i) { return i < nblk ? u.seq_len - (first + W * i) * kBlock : 0; };
 #pragma unroll
       for (int k = 0; k < NSD - 1; ++k) dma_block(min(k, nblk - 1), k, valid_of(k));
       for (int base = 0; base < nblk; base += NSD) {
@@ -890,16 +1008,17 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
     // leaves them in flight (vector loads complete in order).
     u32x4 kf[NL], vf[NL];
     if (nblk > 0) {
-      float pg = page_load(min(1, nblk - 1));
-      const int64_t base0 = block_base(0);
-      load_block(base0, kf, vf, true);
+      auto entry = table_load(min(1, nblk - 1));
+      auto src = first_src(0);
+      load_half(kc, src, kf, true);
+      load_half(vc, src, vf, true);
       for (int i = 0; i < nblk; ++i) {
         const bool more = i + 1 < nblk;
-        const int64_t next = page_base(min(i + 1, nblk - 1), __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, pg)));
-        pg = page_load(min(i + 2, nblk - 1));
+        src = block_src(min(i + 1, nblk - 1), entry);
+        entry = table_load(min(i + 2, nblk - 1));
 #pragma unroll
         for (int c = 0; c < NL; ++c) stage16(kstage + load_tok(c) * KROW + load_dim(c), kf[c]);
-        load_half(kc + next, kf, more);
+        load_half(kc, src, kf, more);
         u32x4 ka[KC];
 #pragma unroll
         for (int c = 0; c < KC; ++c) ka[c] = *reinterpret_cast<const u32x4*>(k_src + 4 * EPC * c);
@@ -917,7 +1036,7 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
               const int h = dt & ~3, e = dt & 3;
               return u32x4{vf[h][e], vf[h + 1][e], vf[h + 2][e], vf[h + 3][e]};
             });
-        load_half(vc + next, vf, more);
+        load_half(vc, src, vf, more);
       }
     }
   } else if (nblk > 0) {
@@ -939,20 +1058,21 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
     // loop, and entries loaded after those K/V would make it wait for them on
     // every iteration.
     u32x4 kb[NS][NL], vb[NS][NL];
-    float pg[NS];  // entry bits of blocks i + NS - 1 .. i + 2NS - 2, slot = block % NS
+    // Entries of blocks i + NS - 1 .. i + 2NS - 2, slot = block % NS.
+    std::conditional_t<SP, Entries, float> pg[NS];
 #pragma unroll
-    for (int k = NS - 1; k < 2 * NS - 1; ++k) pg[k % NS] = page_load(min(k, nblk - 1));
+    for (int k = NS - 1; k < 2 * NS - 1; ++k) pg[k % NS] = table_load(min(k, nblk - 1));
 #pragma unroll
-    for (int s = 0; s < NS - 1; ++s) load_block(block_base(min(s, nblk - 1)), kb[s], vb[s], s < nblk);
+    for (int s = 0; s < NS - 1; ++s) load_block(first_src(min(s, nblk - 1)), kb[s], vb[s], s < nblk);
     for (int base = 0; base < nblk; base += NS) {
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
         const int i = base + s;
         const int slot = (s + NS - 1) % NS;  // block i + NS - 1 (base is a multiple of NS)
         const int j = min(i + NS - 1, nblk - 1);
-        const int64_t nb = page_base(j, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, pg[slot])));
-        pg[slot] = page_load(min(i + 2 * NS - 1, nblk - 1));
-        load_block(nb, kb[slot], vb[slot], i + NS - 1 < nblk);
+        const auto next = block_src(j, pg[slot]);
+        pg[slot] = table_load(min(i + 2 * NS - 1, nblk - 1));
+        load_block(next, kb[slot], vb[slot], i + NS - 1 < nblk);
         process_block(i, kb[s], vb[s]);
       }
     }
@@ -1240,7 +1360,7 @@ __global__ void __launch_bounds__((uniform_waves<E, D, NT>() * 64), (mfma_waves_
   __shared__ __attribute__((
       aligned(16))) char lds[MfmaLds<D, NT, W, dma_staged<KVF, D, NT>(), kDmaStages, E::kBytes>::kBytes];
   __shared__ int s_last[1];
-  fetch_args(a);
+  fetch_args<dma_staged<KVF, D, NT>()>(a);
   // q and the first block-table window depend on the unit alone: they are
   // issued before the kernel waits for seq_lens, so the first K/V loads
   // follow one memory round trip after it instead of two.
@@ -1288,7 +1408,7 @@ __global__ void __launch_bounds__(2 * kThreads, (mfma_waves_per_eu<D, NT>()))
   // Both halves hold the same sequence and split, so they agree on whether
   // there is work, whether it is final and how many segments the unit has:
   // they pass the same workgroup barriers.
-  fetch_args(a);
+  fetch_args<dma_staged<KVF, D, NT>()>(a);
   // q and the first block-table window before seq_lens (decode_mfma_kernel).
   Unit u = decode_unit_paired_ids(a, half);
   QFrag<NT, qk_chunks<E, D>()> q;
@@ -1331,16 +1451,14 @@ __global__ void __launch_bounds__(2 * kThreads, (mfma_waves_per_eu<D, NT>()))
 
 __device__ __forceinline__ int seq_pages(const DecodeArgs& a, int b) {
   const int raw = a.seq_lens[b];
-  const int64_t cap = static_cast<int64_t>(a.max_pages) * a.page_size;
-  const int len = static_cast<int>(raw < cap ? raw : cap);
+  const int len = min(raw, a.max_len);
   return len > 0 ? (len + a.page_size - 1) / a.page_size : 0;
 }
 
 // seq_pages for a wave-uniform b: one scalar load.
 __device__ __forceinline__ int seq_pages_uniform(const DecodeArgs& a, int b) {
   const int raw = as_constant(a.seq_lens)[b];
-  const int64_t cap = static_cast<int64_t>(a.max_pages) * a.page_size;
-  const int len = static_cast<int>(raw < cap ? raw : cap);
+  const int len = min(raw, a.max_len);
   return len > 0 ? (len + a.page_size - 1) / a.page_size : 0;
 }
 
@@ -1425,8 +1543,7 @@ struct Start {
 };
 
 __device__ __forceinline__ int clamped_len(const DecodeArgs& a, int raw) {
-  const int64_t cap = static_cast<int64_t>(a.max_pages) * a.page_size;
-  return static_cast<int>(raw < cap ? raw : cap);
+  return min(raw, a.max_len);
 }
 
 __device__ __forceinline__ int pages_of(const DecodeArgs& a, int len) {
@@ -1622,7 +1739,7 @@ __global__ void __launch_bounds__(PAIR * kThreads, (mfma_waves_per_eu<D, NT>()))
   using Lds = MfmaLds<D, NT, W, dma_staged<KVF, D, NT>()>;
   __shared__ __attribute__((aligned(16))) char lds[PAIR * Lds::kBytes];
   __shared__ int s_last[PAIR];
-  fetch_args(a);
+  fetch_args<dma_staged<KVF, D, NT>()>(a);
   // A compile-time 0 with PAIR == 1, so the LDS base stays a constant.
   const int half = PAIR == 2 ? wave_id() / W : 0;
   const int hp = a.num_kv_heads * a.head_groups / PAIR;  // list units per sequence
@@ -2106,8 +2223,7 @@ __global__ void __launch_bounds__(64) decode_merge_kernel(const DecodeArgs a, in
   const int b = bh / a.num_q_heads;
   const int lane = __lane_id();
   const int raw = a.seq_lens[b];
-  const int64_t cap = static_cast<int64_t>(a.max_pages) * a.page_size;
-  const int seq_len = static_cast<int>(raw < cap ? raw : cap);
+  const int seq_len = min(raw, a.max_len);
   const int num_pages = seq_len > 0 ? (seq_len + a.page_size - 1) / a.page_size : 0;
   const int active = min(a.num_splits, (num_pages + a.pages_per_split - 1) / a.pages_per_split);
   S* out = static_cast<S*>(a.out) + static_cast<int64_t>(bh) * head_dim;
@@ -2252,23 +2368,33 @@ __global__ void __launch_bounds__(64) cascade_merge_kernel(const CascadeArgs c, 
 
 // -------------------------------------------------------------- host side
 
-// Sets the page size and the multiplier / shift of the block -> page
-// division (block_page). With d = blocks per page, l = ceil(log2 d) and
-// p = 31 + l, m = ceil(2^p / d) is below 2^32, and for 0 <= n < 2^31
-// n m / 2^p = n / d + n e / (d 2^p) with e = m d - 2^p in [0, d): the excess
-// is below 2^31 / 2^p = 2^-l <= 1 / d, so the floor is floor(n / d).
-void set_page_size(DecodeArgs& a, int page_size) {
-  a.page_size = page_size;
-  const uint64_t d = static_cast<uint64_t>(std::max(1, page_size / kBlock));
+// The multiplier and shift of a division by d (block_page, table_column). With
+// l = ceil(log2 d) and p = 31 + l, m = ceil(2^p / d) is below 2^32, and for
+// 0 <= n < 2^31 n m / 2^p = n / d + n e / (d 2^p) with e = m d - 2^p in [0, d):
+// the excess is below 2^31 / 2^p = 2^-l <= 1 / d, so the floor is floor(n / d).
+void set_division(int divisor, uint32_t* magic, int* shift) {
+  const uint64_t d = static_cast<uint64_t>(divisor);
   int l = 0;
   while ((uint64_t{1} << l) < d) ++l;
-  a.bpp_shift = 31 + l;
-  a.bpp_magic = static_cast<uint32_t>(((uint64_t{1} << a.bpp_shift) + d - 1) / d);
+  *shift = 31 + l;
+  *magic = static_cast<uint32_t>(((uint64_t{1} << *shift) + d - 1) / d);
+}
+
+// The longest sequence a table of max_pages columns holds.
+int table_tokens(int max_pages, int page_size) {
+  return static_cast<int>(std::min<int64_t>(static_cast<int64_t>(max_pages) * page_size, 0x7fffffff));
+}
+
+// The page sizes: the block table's, and the one the schedule counts in.
+void set_page_size(DecodeArgs& a, int table_page, int schedule_page) {
+  a.page_size = schedule_page;
+  set_division(std::max(1, schedule_page / kBlock), &a.bpp_magic, &a.bpp_shift);
+  a.table_page = table_page;
+  set_division(table_page, &a.table_magic, &a.table_shift);
 }
 
 // Shapes the MFMA kernels serve.
-bool mfma_path(kl_dtype dtype, int head_dim, int page_size) {
-  if (page_size % kBlock != 0) return false;
+bool mfma_path(kl_dtype dtype, int head_dim) {
   if (head_dim == 64 || head_dim == 128 || head_dim == 256) return true;
   // fp32's V operand takes 64 head dims at a time.
   return head_dim == 32 && dtype != KL_DTYPE_F32;
@@ -2490,6 +2616,9 @@ void head_tiling(bool mfma, int head_dim, int group, int* per_wg, int* groups) {
 }
 
 struct Plan {
+  bool mfma;            // MFMA kernels, else the VALU kernel
+  int page_size;        // the page the schedule counts in, and the columns of it
+  int max_pages;        // (the table's own, but for SmallPages: see make_plan)
   int num_splits;       // uniform splits; 0 with the balanced schedule
   int pages_per_split;
   int heads_per_wg;
@@ -2521,7 +2650,21 @@ int make_plan(const Options& opt, kl_dtype dtype, int batch, int num_q_heads, in
   if (dtype != KL_DTYPE_F32 && dtype != KL_DTYPE_F16 && dtype != KL_DTYPE_BF16) {
     return fail(KL_ERR_UNSUPPORTED, "dtype must be f32, f16 or bf16");
   }
-  const bool mfma = use_mfma && mfma_path(dtype, head_dim, page_size);
+  const bool whole_blocks = page_size % kBlock == 0;
+  // Pages that do not hold whole blocks: a split or a workgroup's range is
+  // counted in pages of one block when the planner chooses it, so the rules
+  // below see the lengths they were measured at, and in the table's own pages
+  // when the caller gives the split count, as the original counts them. The
+  // few tables whose length in blocks passes an int keep the VALU kernel.
+  const int64_t blocks = cdiv(static_cast<int64_t>(max_pages) * page_size, kBlock);
+  const bool mfma = use_mfma && mfma_path(dtype, head_dim) && (whole_blocks || blocks <= 0x7fffffff);
+  p->mfma = mfma;
+  if (mfma && !whole_blocks && num_splits <= 0) {
+    page_size = kBlock;
+    max_pages = static_cast<int>(blocks);
+  }
+  p->page_size = page_size;
+  p->max_pages = max_pages;
   const bool mfma16 = mfma && dtype != KL_DTYPE_F32;  // fp32 runs uniform splits, one KV head per workgroup
   if (!mfma && !valu_head_dim_ok(dtype, head_dim)) {
     return fail(KL_ERR_UNSUPPORTED, "head_dim must be 16, 32, 64, 128 or 256");
@@ -2541,7 +2684,7 @@ int make_plan(const Options& opt, kl_dtype dtype, int batch, int num_q_heads, in
   const int64_t pair_units = units / 2;
   const bool long_pairs = pair_units * pages >= static_cast<int64_t>(cus) * kPairMinPages &&
                           pair_units * kPairMaxSegments >= cus;
-  const bool pairable = mfma16 && !partials && opt.pairing() && num_kv_heads % 2 == 0 && head_dim <= 128 &&
+  const bool pairable = mfma16 && whole_blocks && !partials && opt.pairing() && num_kv_heads % 2 == 0 && head_dim <= 128 &&
                         p->heads_per_wg <= 16 && (units >= 2 * static_cast<int64_t>(cus) || long_pairs);
   // Batches whose units fill the device (units >= CUs) take the balanced
   // schedule too. The planner cannot see seq_lens, and with uniform splits
@@ -2656,7 +2799,7 @@ int make_plan(const Options& opt, kl_dtype dtype, int batch, int num_q_heads, in
   // Two adjacent KV heads per 8-wave workgroup when the pairs alone give
   // every CU a workgroup (one 8-wave workgroup per CU is the register budget)
   // and the 4-wave kernel fits two waves per SIMD (head_dim <= 128).
-  p->paired = mfma16 && opt.pairing() && num_kv_heads % 2 == 0 && head_dim <= 128 && units * s / 2 >= cus;
+  p->paired = mfma16 && whole_blocks && opt.pairing() && num_kv_heads % 2 == 0 && head_dim <= 128 && units * s / 2 >= cus;
   if (s > 1 || partials) {
     const size_t rows = static_cast<size_t>(batch) * num_q_heads * s;
     p->o_bytes = align_up(rows * head_dim * sizeof(float));
@@ -2771,11 +2914,12 @@ int launch_uniform_mfma(const DecodeArgs& a, int head_dim, unsigned grid, hipStr
     if constexpr (mfma_instance_exists<KVF, D>()) {
       if (a.paired) {
         // head_dim 256 and fp32 are never paired: the segment needs more than
-        // the 256 registers per lane an 8-wave workgroup leaves.
-        if constexpr (D <= 128 && !std::is_same_v<E, F32>) {
+        // the 256 registers per lane an 8-wave workgroup leaves. Small pages
+        // are not paired either (make_plan).
+        if constexpr (D <= 128 && !std::is_same_v<E, F32> && !kSmallPages<KVF>) {
           decode_mfma_paired_kernel<E, KVF, D, NT><<<grid / 2, 2 * kThreads, 0, stream>>>(a);
         } else {
-          return fail(KL_ERR_UNSUPPORTED, "paired decode needs 16-bit queries and head_dim <= 128");
+          return fail(KL_ERR_UNSUPPORTED, "paired decode needs 16-bit queries, whole blocks per page and head_dim <= 128");
         }
       } else {
         decode_mfma_kernel<E, KVF, D, NT><<<grid, uniform_waves<E, D, NT>() * 64, 0, stream>>>(a);
@@ -2816,7 +2960,7 @@ int launch_balanced(DecodeArgs a, int head_dim, hipStream_t stream) {
       if (a.paired) {
         // One head tile and head_dim <= 128: beyond that the segment needs
         // more than the 256 registers per lane of an 8-wave workgroup.
-        if constexpr (D <= 128 && NT == 1) {
+        if constexpr (D <= 128 && NT == 1 && !kSmallPages<KVF>) {
           decode_mfma_balanced_kernel<E, KVF, D, NT, 2><<<grid, 2 * kThreads, 0, stream>>>(a);
         } else {
           return fail(KL_ERR_UNSUPPORTED, "paired balanced decode needs head_dim <= 128 and <= 16 heads per workgroup");
@@ -2901,7 +3045,7 @@ int decode_entry(kl_dtype dtype, bool kv8, void* out, const void* q, const void*
     if (dtype != KL_DTYPE_F16 && dtype != KL_DTYPE_BF16) {
       return fail(KL_ERR_UNSUPPORTED, "an FP8 cache needs fp16 or bf16 queries");
     }
-    if (!mfma_path(dtype, head_dim, page_size) || head_dim < 64) {
+    if (!mfma_path(dtype, head_dim) || page_size % kBlock != 0 || head_dim < 64) {
       return fail(KL_ERR_UNSUPPORTED, "an FP8 cache needs head_dim 64, 128 or 256 and page_size a multiple of 16");
     }
     if (!k_scale || !v_scale) return fail(KL_ERR_INVALID_ARGUMENT, "k_scale and v_scale must be non-null");
@@ -2951,8 +3095,9 @@ int decode_entry(kl_dtype dtype, bool kv8, void* out, const void* q, const void*
   a.num_q_heads = num_q_heads;
   a.num_kv_heads = num_kv_heads;
   a.group = num_q_heads / num_kv_heads;
-  set_page_size(a, page_size);
-  a.max_pages = max_pages;
+  set_page_size(a, page_size, p.page_size);
+  a.max_pages = p.max_pages;
+  a.max_len = table_tokens(max_pages, page_size);
   a.num_splits = p.num_splits;
   a.pages_per_split = p.pages_per_split;
   a.head_groups = p.head_groups;
@@ -2967,16 +3112,19 @@ int decode_entry(kl_dtype dtype, bool kv8, void* out, const void* q, const void*
   a.paired = p.paired ? 1 : 0;
   a.arrivals = nullptr;
 
-  const bool mfma = use_mfma && mfma_path(dtype, head_dim, page_size);
+  const bool small_pages = p.mfma && page_size % kBlock != 0;
   switch (dtype) {
     case KL_DTYPE_F32:
-      return launch_typed<F32, F32>(a, head_dim, mfma, stream);
+      return small_pages ? launch_typed<F32, SmallPages<F32>>(a, head_dim, true, stream)
+                         : launch_typed<F32, F32>(a, head_dim, p.mfma, stream);
     case KL_DTYPE_F16:
-      return kv8 ? launch_typed<F16, Fp8E4M3>(a, head_dim, true, stream)
-                 : launch_typed<F16, F16>(a, head_dim, mfma, stream);
+      return kv8           ? launch_typed<F16, Fp8E4M3>(a, head_dim, true, stream)
+             : small_pages ? launch_typed<F16, SmallPages<F16>>(a, head_dim, true, stream)
+                           : launch_typed<F16, F16>(a, head_dim, p.mfma, stream);
     case KL_DTYPE_BF16:
-      return kv8 ? launch_typed<BF16, Fp8E4M3>(a, head_dim, true, stream)
-                 : launch_typed<BF16, BF16>(a, head_dim, mfma, stream);
+      return kv8           ? launch_typed<BF16, Fp8E4M3>(a, head_dim, true, stream)
+             : small_pages ? launch_typed<BF16, SmallPages<BF16>>(a, head_dim, true, stream)
+                           : launch_typed<BF16, BF16>(a, head_dim, p.mfma, stream);
   }
   return fail(KL_ERR_UNSUPPORTED, "dtype must be f32, f16 or bf16");
 }
@@ -3116,7 +3264,7 @@ int cascade_plan(kl_dtype dtype, int batch, int num_q_heads, int num_kv_heads, i
   if (dtype != KL_DTYPE_F16 && dtype != KL_DTYPE_BF16) {
     return fail(KL_ERR_UNSUPPORTED, "cascade decode needs fp16 or bf16");
   }
-  if (!mfma_path(dtype, head_dim, page_size)) {
+  if (!mfma_path(dtype, head_dim) || page_size % kBlock != 0) {
     return fail(KL_ERR_UNSUPPORTED, "cascade decode needs head_dim 32, 64, 128 or 256 and page_size a multiple of 16");
   }
   if (batch < 0 || num_kv_heads <= 0 || num_q_heads <= 0 || prefix_pages < 0 || max_pages < 0) {
@@ -3155,6 +3303,7 @@ int cascade_launch(const DecodeArgs& base, const CascadePlan& cp, const int32_t*
     a.group = batch * group;
     a.num_q_heads = a.num_kv_heads * a.group;
     a.max_pages = prefix_pages;
+    a.max_len = table_tokens(prefix_pages, a.page_size);
     a.num_splits = cp.pre.num_splits;
     a.pages_per_split = cp.pre.pages_per_split;
     a.head_groups = cp.pre.head_groups;
@@ -3174,6 +3323,7 @@ int cascade_launch(const DecodeArgs& base, const CascadePlan& cp, const int32_t*
   a.seq_lens = seq_lens;
   a.bt_stride = bt_stride;
   a.max_pages = max_pages;
+  a.max_len = table_tokens(max_pages, a.page_size);
   a.num_splits = cp.suf.num_splits;
   a.pages_per_split = cp.suf.pages_per_split;
   a.head_groups = cp.suf.head_groups;
@@ -3272,7 +3422,7 @@ extern "C" int kl_cascade_decode_attention(kl_dtype dtype, void* out, const void
   a.num_q_heads = num_q_heads;
   a.num_kv_heads = num_kv_heads;
   a.group = num_q_heads / num_kv_heads;
-  set_page_size(a, page_size);
+  set_page_size(a, page_size, page_size);
   a.grid = 0;
   a.paired = 0;
   a.arrivals = nullptr;
