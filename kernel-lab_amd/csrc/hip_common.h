@@ -122,6 +122,7 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
 // row_ror:n rotates the 16 lanes of each row by n.
 constexpr int kDppQuadSwap1 = 0xB1;  // quad_perm [1,0,3,2]: lane ^ 1
 constexpr int kDppQuadSwap2 = 0x4E;  // quad_perm [2,3,0,1]: lane ^ 2
+constexpr int kDppRowHalfMirror = 0x141;  // reverses each 8 lanes
 constexpr int kDppRowRor4 = 0x124;
 constexpr int kDppRowRor8 = 0x128;
 // row_shr:n moves lane i's value to lane i + n of the same 16-lane row.

@@ -8,15 +8,21 @@
 // that rounded value is what the residual stream keeps; the residual output is
 // therefore bit-identical to PyTorch's.
 //
-// Design: one workgroup per row. Each thread loads its share of the row as
-// 16-byte packs, strided by the workgroup size so every wave load is one
-// contiguous 1 KiB span, and keeps the values in registers. The sum of squares
-// is reduced within each wave by DPP, across waves through LDS with one
-// barrier, and the output is written from registers: one read of x and the
-// residual, one write of the residual and the output, nothing re-read.
-// Rows too wide for the register budget use a two-pass variant that keeps the
-// rounded sum in LDS (and forms it again for what LDS cannot hold).
+// Design: one workgroup per row, several rows per workgroup where a row is
+// narrow. Each thread loads its share of the row as 16-byte packs, strided by
+// the row's threads so every wave load is contiguous, and keeps the values in
+// registers. The sum of squares is reduced within each wave by DPP, across
+// waves (if the row has several) through LDS with one barrier, and the output
+// is written from registers: one read of x and the residual, one write of the
+// residual and the output, nothing re-read.
+//   rms_norm_reg_kernel     wide rows, 16-byte aligned
+//   rms_norm_rows_kernel    narrow rows: a row per 4 .. 64 lanes
+//   rms_norm_ragged_kernel  wide rows at any address and width
+//   rms_norm_staged_kernel  rows too wide for the register budget: two passes,
+//                           the rounded sum kept in LDS (and formed again for
+//                           what LDS cannot hold)
 #include <algorithm>
+#include <type_traits>
 
 #include "hip_common.h"
 #include "kl_internal.h"
@@ -49,6 +55,121 @@ __device__ __forceinline__ void store_pack(Pack<S, N>* p, const Pack<S, N>& v) {
 
 constexpr int kMaxThreads = 1024;
 
+__device__ __forceinline__ float inv_rms(float sum_sq, int hidden, float eps) {
+  // Division and square root are IEEE-rounded here (no fast-math), matching
+  // torch.rsqrt on the CPU, which computes 1 / sqrt(x).
+  return 1.0f / sqrtf(sum_sq / static_cast<float>(hidden) + eps);
+}
+
+// The 16 bytes at element offset `off` of a row. Unaligned rows (any element
+// alignment) use the same 16-byte memory instructions, which gfx950 takes at
+// any address.
+template <bool ALIGNED, typename P, typename S>
+__device__ __forceinline__ P load_at(const S* row, int off) {
+  P v;
+  if constexpr (ALIGNED) {
+    v = *reinterpret_cast<const P*>(row + off);
+  } else {
+    __builtin_memcpy(&v, row + off, sizeof(P));
+  }
+  return v;
+}
+template <bool ALIGNED, typename P, typename S>
+__device__ __forceinline__ void store_at(S* row, int off, const P& v) {
+  if constexpr (ALIGNED) {
+    *reinterpret_cast<P*>(row + off) = v;
+  } else {
+    __builtin_memcpy(row + off, &v, sizeof(P));
+  }
+}
+
+// One thread's share of a row: packs t, t + nt, ..., NPACK of them, held in
+// registers. reduce(v) sums v over the row's threads. live false: a row past
+// the last, loaded like the last and not stored.
+//
+// ALIGNED: every row starts on 16 bytes and holds whole packs. Otherwise the
+// last pack is the row's last VEC elements, which overlap the pack before it
+// when the width is not a multiple of VEC: it leaves those elements out of the
+// sum and writes the same values to them. The residual is updated in place, so
+// without ALIGNED it is stored after the reduction, which every thread of the
+// row reaches with its loads done.
+template <typename E, int VEC, int NPACK, bool HAS_RES, bool ALIGNED, typename Reduce>
+__device__ __forceinline__ void norm_row(typename E::S* out, const typename E::S* x, typename E::S* res,
+                                         const typename E::S* weight, int hidden, float eps, int t, int nt, bool live,
+                                         Reduce&& reduce) {
+  using S = typename E::S;
+  using P = Pack<S, VEC>;
+  const int packs = ALIGNED ? hidden / VEC : (hidden + VEC - 1) / VEC;
+  int off[NPACK];
+  int skip[NPACK];  // leading elements of the pack that the one before it holds
+  bool valid[NPACK];
+#pragma unroll
+  for (int k = 0; k < NPACK; ++k) {
+    const int p = t + k * nt;
+    valid[k] = p < packs;
+    const int at = (valid[k] ? p : packs - 1) * VEC;
+    off[k] = ALIGNED ? at : min(at, hidden - VEC);
+    skip[k] = at - off[k];
+  }
+  P a[NPACK], b[NPACK], w[NPACK];
+#pragma unroll
+  for (int k = 0; k < NPACK; ++k) {
+    a[k] = load_at<ALIGNED, P>(x, off[k]);
+    if constexpr (HAS_RES) b[k] = load_at<ALIGNED, P>(res, off[k]);
+  }
+  // As in rms_norm_reg_kernel: ahead of the reduction unless the registers are short.
+  constexpr bool kEarlyWeights = NPACK <= 4;
+  if constexpr (kEarlyWeights) {
+#pragma unroll
+    for (int k = 0; k < NPACK; ++k) w[k] = load_at<ALIGNED, P>(weight, off[k]);
+  }
+  float sum_sq = 0.0f;
+#pragma unroll
+  for (int k = 0; k < NPACK; ++k) {
+    float part = 0.0f;
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      if constexpr (HAS_RES) a[k].v[j] = E::from_f32(E::to_f32(a[k].v[j]) + E::to_f32(b[k].v[j]));
+      const float f = E::to_f32(a[k].v[j]);
+      part += ALIGNED || j >= skip[k] ? f * f : 0.0f;
+    }
+    sum_sq += valid[k] ? part : 0.0f;
+  }
+  if constexpr (HAS_RES && ALIGNED) {
+#pragma unroll
+    for (int k = 0; k < NPACK; ++k) {
+      if (valid[k] && live) store_at<ALIGNED>(res, off[k], a[k]);
+    }
+  }
+  const float rstd = inv_rms(reduce(sum_sq), hidden, eps);
+  if constexpr (HAS_RES && !ALIGNED) {
+#pragma unroll
+    for (int k = 0; k < NPACK; ++k) {
+      if (valid[k] && live) store_at<ALIGNED>(res, off[k], a[k]);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < NPACK; ++k) {
+    if constexpr (!kEarlyWeights) w[k] = load_at<ALIGNED, P>(weight, off[k]);
+    P o;
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) o.v[j] = E::from_f32((E::to_f32(a[k].v[j]) * rstd) * E::to_f32(w[k].v[j]));
+    if (valid[k] && live) store_at<ALIGNED>(out, off[k], o);
+  }
+}
+
+// Sum over the LANES (4 .. 64) lanes of a row, in every one of them.
+template <int LANES>
+__device__ __forceinline__ float lanes_sum(float v) {
+  v += dpp<kDppQuadSwap1>(v);
+  v += dpp<kDppQuadSwap2>(v);
+  if constexpr (LANES >= 8) v += dpp<kDppRowHalfMirror>(v);  // the quads of each half row agree, so a mirror is a swap
+  if constexpr (LANES >= 16) v += dpp<kDppRowRor8>(v);
+  if constexpr (LANES >= 32) v = sum_xor16(v);
+  if constexpr (LANES >= 64) v = sum_xor32(v);
+  return v;
+}
+
 // Workgroup-wide sum; every thread receives the same value. `scratch` holds one
 // float per wave. Wave sums are added in wave order, so the result is
 // deterministic.
@@ -60,12 +181,6 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
   float total = 0.0f;
   for (int i = 0; i < nw; ++i) total += scratch[i];
   return total;
-}
-
-__device__ __forceinline__ float inv_rms(float sum_sq, int hidden, float eps) {
-  // Division and square root are IEEE-rounded here (no fast-math), matching
-  // torch.rsqrt on the CPU, which computes 1 / sqrt(x).
-  return 1.0f / sqrtf(sum_sq / static_cast<float>(hidden) + eps);
 }
 
 // Register-resident single pass. Thread t owns packs t, t + NT, ..., so NPACK
@@ -246,48 +361,139 @@ __global__ void __launch_bounds__(kMaxThreads)
   }
 }
 
+// Rows of at most kRowsMaxPacks packs: LANES lanes per row and 256 / LANES rows
+// per workgroup, so a narrow row neither leaves lanes idle nor costs a
+// workgroup of its own, and the reduction stays in a wave (no barrier). What
+// bounds it: memory for many rows, the launch for few. Measured, a workgroup
+// per row -> this (us, bf16): 65,536 rows of 128 16.9 -> 6.9 (4.9 TB/s), of 64
+// 16.6 -> 4.6, 16,384 rows of 512 7.2 -> 6.8; 16 rows of 128 equal.
+constexpr int kRowsThreads = 256;
+
+template <typename E, int LANES, int NPACK, bool HAS_RES, bool ALIGNED>
+__global__ void __launch_bounds__(kRowsThreads)
+    rms_norm_rows_kernel(typename E::S* __restrict__ out, const typename E::S* __restrict__ x,
+                         typename E::S* __restrict__ res, const typename E::S* __restrict__ weight, int rows, int hidden, int64_t x_row_stride, float eps) {
+  const int64_t r = static_cast<int64_t>(blockIdx.x) * (kRowsThreads / LANES) + threadIdx.x / LANES;
+  const bool live = r < rows;
+  const int64_t row = live ? r : rows - 1;
+  norm_row<E, 16 / E::kBytes, NPACK, HAS_RES, ALIGNED>(
+      out + row * hidden, x + row * x_row_stride, HAS_RES ? res + row * hidden : nullptr, weight, hidden, eps,
+      threadIdx.x % LANES, LANES, live, [](float v) { return lanes_sum<LANES>(v); });
+}
+
+// Wide rows whose width or addresses are not multiples of 16 bytes: one
+// workgroup per row on unaligned 16-byte accesses, in place of element-wide
+// ones. Memory bounds it. Measured, element-wide -> this (us): add + norm 4,096
+// rows of 5,003 bf16 54.5 -> 35.4, 2,048 of 4,099 fp32 30.7 -> 24.8, norm of
+// 2,048 of 4,099 fp16 12.1 -> 8.8.
+template <typename E, int NPACK, bool HAS_RES>
+__global__ void __launch_bounds__(kMaxThreads)
+    rms_norm_ragged_kernel(typename E::S* __restrict__ out, const typename E::S* __restrict__ x,
+                           typename E::S* __restrict__ res, const typename E::S* __restrict__ weight, int hidden, int64_t x_row_stride, float eps) {
+  __shared__ float scratch[kMaxThreads / 64];
+  const int64_t row = blockIdx.x;
+  norm_row<E, 16 / E::kBytes, NPACK, HAS_RES, false>(
+      out + row * hidden, x + row * x_row_stride, HAS_RES ? res + row * hidden : nullptr, weight, hidden, eps,
+      threadIdx.x, blockDim.x, true, [&](float v) { return block_sum(v, scratch); });
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-template <typename E, int VEC, bool HAS_RES>
-int launch_vec(void* out, const void* x, void* res, const void* w, int64_t rows, int hidden,
-               int64_t x_row_stride, float eps, hipStream_t stream) {
+// Calls f(IntC<N>) with the smallest N of 1, 2, 4, 8 that holds npack.
+template <int N>
+using IntC = std::integral_constant<int, N>;
+template <typename F>
+void with_packs(int npack, F&& f) {
+  if (npack <= 1) {
+    f(IntC<1>{});
+  } else if (npack <= 2) {
+    f(IntC<2>{});
+  } else if (npack <= 4) {
+    f(IntC<4>{});
+  } else {
+    f(IntC<8>{});
+  }
+}
+
+// Widest row, in packs, that rms_norm_rows_kernel takes: a pack per lane of one
+// wave. With two packs a lane it lost to a workgroup per row (8,192 rows of
+// 1,024 bf16: 7.5 against 6.7 us).
+constexpr int kRowsMaxPacks = 64;
+
+template <typename E, bool HAS_RES>
+int launch_typed(void* out, const void* x, void* res, const void* w, int64_t rows, int hidden,
+                 int64_t x_row_stride, float eps, hipStream_t stream) {
   using S = typename E::S;
+  constexpr int VEC = 16 / E::kBytes;
   auto* o = static_cast<S*>(out);
   auto* xi = static_cast<const S*>(x);
   auto* r = static_cast<S*>(res);
   auto* wi = static_cast<const S*>(w);
-  const int packs = hidden / VEC;
-  // About kPacksPerThread packs per thread, in whole waves, 64..1024 threads.
-  int threads = static_cast<int>(std::min<int64_t>(
-      kMaxThreads, std::max<int64_t>(64, cdiv(cdiv(packs, kPacksPerThread), 64) * 64)));
-  const int npack = static_cast<int>(cdiv(packs, threads));
+  const bool aligned = hidden % VEC == 0 && x_row_stride % VEC == 0 && aligned16(out) && aligned16(x) &&
+                       aligned16(w) && (res == nullptr || aligned16(res));
+  const int packs = static_cast<int>(cdiv(hidden, VEC));
   const dim3 grid(static_cast<unsigned>(rows));
-  if (npack <= 1) {
-    rms_norm_reg_kernel<E, VEC, 1, HAS_RES><<<grid, threads, 0, stream>>>(o, xi, r, wi, hidden, x_row_stride, eps);
-  } else if (npack <= 2) {
-    rms_norm_reg_kernel<E, VEC, 2, HAS_RES><<<grid, threads, 0, stream>>>(o, xi, r, wi, hidden, x_row_stride, eps);
-  } else if (npack <= 4) {
-    rms_norm_reg_kernel<E, VEC, 4, HAS_RES><<<grid, threads, 0, stream>>>(o, xi, r, wi, hidden, x_row_stride, eps);
-  } else if (npack <= 8) {
-    rms_norm_reg_kernel<E, VEC, 8, HAS_RES><<<grid, threads, 0, stream>>>(o, xi, r, wi, hidden, x_row_stride, eps);
+  if (hidden < VEC) {  // less than a pack: element by element
+    rms_norm_reg_kernel<E, 1, 1, HAS_RES><<<grid, 64, 0, stream>>>(o, xi, r, wi, hidden, x_row_stride, eps);
+    return check_launch("rms_norm kernel launch");
+  }
+  if (packs <= kRowsMaxPacks) {
+    auto rows_kernel = [&](auto lanes, auto np) {
+      constexpr int L = decltype(lanes)::value, NP = decltype(np)::value;
+      const unsigned wgs = static_cast<unsigned>(cdiv(rows, kRowsThreads / L));
+      if (aligned) {
+        rms_norm_rows_kernel<E, L, NP, HAS_RES, true><<<wgs, kRowsThreads, 0, stream>>>(
+            o, xi, r, wi, static_cast<int>(rows), hidden, x_row_stride, eps);
+      } else {
+        rms_norm_rows_kernel<E, L, NP, HAS_RES, false><<<wgs, kRowsThreads, 0, stream>>>(
+            o, xi, r, wi, static_cast<int>(rows), hidden, x_row_stride, eps);
+      }
+    };
+    if (packs <= 4) {
+      rows_kernel(IntC<4>{}, IntC<1>{});
+    } else if (packs <= 8) {
+      rows_kernel(IntC<8>{}, IntC<1>{});
+    } else if (packs <= 16) {
+      rows_kernel(IntC<16>{}, IntC<1>{});
+    } else if (packs <= 32) {
+      rows_kernel(IntC<32>{}, IntC<1>{});
+    } else {
+      rows_kernel(IntC<64>{}, IntC<1>{});
+    }
+    return check_launch("rms_norm kernel launch");
+  }
+  // About kPacksPerThread packs per thread, in whole waves, 64..1024 threads.
+  const int threads = static_cast<int>(
+      std::min<int64_t>(kMaxThreads, std::max<int64_t>(64, cdiv(cdiv(packs, kPacksPerThread), 64) * 64)));
+  const int npack = static_cast<int>(cdiv(packs, threads));
+  if (npack > (aligned ? 8 : 4)) {  // eight unaligned packs of x and the residual would spill
+    if (aligned) {
+      rms_norm_staged_kernel<E, VEC, HAS_RES>
+          <<<grid, kMaxThreads, 0, stream>>>(o, xi, r, wi, hidden, x_row_stride, eps);
+    } else {
+      rms_norm_staged_kernel<E, 1, HAS_RES>
+          <<<grid, kMaxThreads, 0, stream>>>(o, xi, r, wi, hidden, x_row_stride, eps);
+    }
   } else {
-    rms_norm_staged_kernel<E, VEC, HAS_RES><<<grid, kMaxThreads, 0, stream>>>(o, xi, r, wi, hidden, x_row_stride, eps);
+    with_packs(npack, [&](auto np) {
+      constexpr int NP = decltype(np)::value;
+      if (aligned) {
+        rms_norm_reg_kernel<E, VEC, NP, HAS_RES>
+            <<<grid, threads, 0, stream>>>(o, xi, r, wi, hidden, x_row_stride, eps);
+      } else if constexpr (NP <= 4) {
+        rms_norm_ragged_kernel<E, NP, HAS_RES>
+            <<<grid, threads, 0, stream>>>(o, xi, r, wi, hidden, x_row_stride, eps);
+      }
+    });
   }
   return check_launch("rms_norm kernel launch");
 }
 
 template <typename E>
-int launch_typed(void* out, const void* x, void* res, const void* w, int64_t rows, int hidden,
-                 int64_t x_row_stride, float eps, hipStream_t stream) {
-  constexpr int kVec = 16 / E::kBytes;
-  const bool vec = hidden % kVec == 0 && x_row_stride % kVec == 0 && aligned16(out) && aligned16(x) &&
-                   aligned16(w) && (res == nullptr || aligned16(res));
-  if (vec) {
-    return res ? launch_vec<E, kVec, true>(out, x, res, w, rows, hidden, x_row_stride, eps, stream)
-               : launch_vec<E, kVec, false>(out, x, res, w, rows, hidden, x_row_stride, eps, stream);
-  }
-  return res ? launch_vec<E, 1, true>(out, x, res, w, rows, hidden, x_row_stride, eps, stream)
-             : launch_vec<E, 1, false>(out, x, res, w, rows, hidden, x_row_stride, eps, stream);
+int launch_any(void* out, const void* x, void* res, const void* w, int64_t rows, int hidden, int64_t x_row_stride,
+               float eps, hipStream_t stream) {
+  return res ? launch_typed<E, true>(out, x, res, w, rows, hidden, x_row_stride, eps, stream)
+             : launch_typed<E, false>(out, x, res, w, rows, hidden, x_row_stride, eps, stream);
 }
 
 }  // namespace
@@ -311,11 +517,11 @@ extern "C" int kl_rms_norm(kl_dtype dtype, void* out, const void* x, void* resid
   const int h = static_cast<int>(hidden);
   switch (dtype) {
     case KL_DTYPE_F32:
-      return launch_typed<F32>(out, x, residual, weight, rows, h, x_row_stride, eps, s);
+      return launch_any<F32>(out, x, residual, weight, rows, h, x_row_stride, eps, s);
     case KL_DTYPE_F16:
-      return launch_typed<F16>(out, x, residual, weight, rows, h, x_row_stride, eps, s);
+      return launch_any<F16>(out, x, residual, weight, rows, h, x_row_stride, eps, s);
     case KL_DTYPE_BF16:
-      return launch_typed<BF16>(out, x, residual, weight, rows, h, x_row_stride, eps, s);
+      return launch_any<BF16>(out, x, residual, weight, rows, h, x_row_stride, eps, s);
   }
   return fail(KL_ERR_UNSUPPORTED, "dtype must be f32, f16 or bf16");
 }
