@@ -90,6 +90,20 @@ int kl_rms_norm(kl_dtype dtype, void* out, const void* x, void* residual, const 
                 kl_stream_t stream);
 
 /*
+ * kl_rms_norm over groups of rows, with the new residual written apart from
+ * the old one. Row i of group g of `x` starts at x + g * x_group_stride + i *
+ * x_row_stride elements (both strides >= hidden), which reads the heads of one
+ * part of a fused projection in place; the other tensors are contiguous over
+ * groups * rows_per_group rows. `residual` and `residual_out` are both null or
+ * both given; they may be the same array (kl_rms_norm's in-place form) and
+ * must not overlap otherwise. No counterpart in the reference, whose wrapper
+ * clones the residual first (kernel_lab/cuda_ops.py:31-61).
+ */
+int kl_rms_norm_grouped(kl_dtype dtype, void* out, const void* x, const void* residual, void* residual_out,
+                        const void* weight, int64_t groups, int64_t rows_per_group, int64_t hidden,
+                        int64_t x_group_stride, int64_t x_row_stride, float eps, kl_stream_t stream);
+
+/*
  * Split planning for paged decode. Pure host arithmetic: it reads no device
  * memory (in particular not seq_lens), so it never synchronises.
  * Follows choose_num_splits and the split normalisation of
@@ -112,7 +126,9 @@ int kl_rms_norm(kl_dtype dtype, void* out, const void* x, void* residual, const 
  *                    detected on the device; full batches of more than 8
  *                    query heads per KV head take it only when the table
  *                    spans >= 256 pages; a single sequence takes uniform
- *                    splits of >= 8 pages)
+ *                    splits of >= 8 pages); when page_size is
+ *                    not a multiple of 16 the planner counts pages of
+ *                    16 tokens, a count the caller gives its own pages
  *   out_workspace    (host pointer) bytes of device workspace the launch needs
  *                    (0 when the launch needs none)
  */

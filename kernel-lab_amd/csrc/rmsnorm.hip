@@ -55,10 +55,43 @@ __device__ __forceinline__ void store_pack(Pack<S, N>* p, const Pack<S, N>& v) {
 
 constexpr int kMaxThreads = 1024;
 
+// Where x's rows are, in elements: row i of group g at g * group_stride + i *
+// row_stride, inner rows to a group; out and the residuals hold row g * inner +
+// i there. A strided view of two leading dimensions (the heads of one part of a
+// fused projection) is read in place; copied first, 2,048 x 32 heads of 128
+// bf16 took 15.7 us, the copy 9.7 of them, and 7.1 read in place.
+//
+// A workgroup per row takes (i, g) from the grid, the larger of the two counts
+// along x: a division before the first load cost the large sizes 2 %.
+struct RowMap {
+  int64_t inner, row_stride, group_stride;
+  int swapped;  // the grid's x counts groups
+  __device__ __forceinline__ void of_workgroup(int64_t* row, int64_t* x_off) const {
+    const int64_t i = swapped ? blockIdx.y : blockIdx.x;
+    const int64_t g = swapped ? blockIdx.x : blockIdx.y;
+    *row = g * inner + i;
+    *x_off = g * group_stride + i * row_stride;
+  }
+  __device__ __forceinline__ int64_t x_of_row(int64_t r) const {
+    if (group_stride == 0) return r * row_stride;  // one group
+    const uint32_t g = static_cast<uint32_t>(r) / static_cast<uint32_t>(inner);
+    return g * group_stride + (r - g * inner) * row_stride;
+  }
+};
+
 __device__ __forceinline__ float inv_rms(float sum_sq, int hidden, float eps) {
   // Division and square root are IEEE-rounded here (no fast-math), matching
   // torch.rsqrt on the CPU, which computes 1 / sqrt(x).
   return 1.0f / sqrtf(sum_sq / static_cast<float>(hidden) + eps);
+}
+
+// The new residual's place, `bytes` past the old one's: 0 in place. Reached
+// from the same pointer, so that pointer can be __restrict__ in both forms
+// (without it the large sizes lost 1 %: the weights' loads went ahead of the
+// residual's).
+template <typename S>
+__device__ __forceinline__ S* residual_out(S* res, int64_t bytes) {
+  return reinterpret_cast<S*>(reinterpret_cast<char*>(res) + bytes);
 }
 
 // The 16 bytes at element offset `off` of a row. Unaligned rows (any element
@@ -90,13 +123,13 @@ __device__ __forceinline__ void store_at(S* row, int off, const P& v) {
 // ALIGNED: every row starts on 16 bytes and holds whole packs. Otherwise the
 // last pack is the row's last VEC elements, which overlap the pack before it
 // when the width is not a multiple of VEC: it leaves those elements out of the
-// sum and writes the same values to them. The residual is updated in place, so
-// without ALIGNED it is stored after the reduction, which every thread of the
-// row reaches with its loads done.
+// sum and writes the same values to them. The residual may be updated in place
+// (res_out 0), so without ALIGNED it is stored after the reduction, which
+// every thread of the row reaches with its loads done.
 template <typename E, int VEC, int NPACK, bool HAS_RES, bool ALIGNED, typename Reduce>
 __device__ __forceinline__ void norm_row(typename E::S* out, const typename E::S* x, typename E::S* res,
-                                         const typename E::S* weight, int hidden, float eps, int t, int nt, bool live,
-                                         Reduce&& reduce) {
+                                         int64_t res_out, const typename E::S* weight, int hidden, float eps,
+                                         int t, int nt, bool live, Reduce&& reduce) {
   using S = typename E::S;
   using P = Pack<S, VEC>;
   const int packs = ALIGNED ? hidden / VEC : (hidden + VEC - 1) / VEC;
@@ -138,14 +171,14 @@ __device__ __forceinline__ void norm_row(typename E::S* out, const typename E::S
   if constexpr (HAS_RES && ALIGNED) {
 #pragma unroll
     for (int k = 0; k < NPACK; ++k) {
-      if (valid[k] && live) store_at<ALIGNED>(res, off[k], a[k]);
+      if (valid[k] && live) store_at<ALIGNED>(residual_out(res, res_out), off[k], a[k]);
     }
   }
   const float rstd = inv_rms(reduce(sum_sq), hidden, eps);
   if constexpr (HAS_RES && !ALIGNED) {
 #pragma unroll
     for (int k = 0; k < NPACK; ++k) {
-      if (valid[k] && live) store_at<ALIGNED>(res, off[k], a[k]);
+      if (valid[k] && live) store_at<ALIGNED>(residual_out(res, res_out), off[k], a[k]);
     }
   }
 #pragma unroll
@@ -192,17 +225,19 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
 template <typename E, int VEC, int NPACK, bool HAS_RES>
 __global__ void __launch_bounds__(kMaxThreads)
     rms_norm_reg_kernel(typename E::S* __restrict__ out, const typename E::S* __restrict__ x,
-                        typename E::S* __restrict__ res, const typename E::S* __restrict__ weight,
-                        int hidden, int64_t x_row_stride, float eps) {
+                        typename E::S* __restrict__ res, int64_t res_out, const typename E::S* __restrict__ weight,
+                        int hidden, RowMap x_rows, float eps) {
   using S = typename E::S;
   using P = Pack<S, VEC>;
   __shared__ float scratch[kMaxThreads / 64];
 
-  const int64_t row = blockIdx.x;
+  int64_t row, x_off;
+  x_rows.of_workgroup(&row, &x_off);
   const int packs = hidden / VEC;
   const int nt = blockDim.x;
-  const P* xr = reinterpret_cast<const P*>(x + row * x_row_stride);
+  const P* xr = reinterpret_cast<const P*>(x + x_off);
   P* rr = HAS_RES ? reinterpret_cast<P*>(res + row * static_cast<int64_t>(hidden)) : nullptr;
+  P* rw = HAS_RES ? residual_out(rr, res_out) : nullptr;
   P* orow = reinterpret_cast<P*>(out + row * static_cast<int64_t>(hidden));
   const P* wr = reinterpret_cast<const P*>(weight);
 
@@ -256,7 +291,7 @@ __global__ void __launch_bounds__(kMaxThreads)
   if constexpr (HAS_RES) {
 #pragma unroll
     for (int k = 0; k < NPACK; ++k) {
-      if (valid[k]) store_pack(rr + idx[k], s[k]);
+      if (valid[k]) store_pack(rw + idx[k], s[k]);
     }
   }
 
@@ -303,19 +338,21 @@ constexpr int kStageBytes = 48 * 1024;
 template <typename E, int VEC, bool HAS_RES>
 __global__ void __launch_bounds__(kMaxThreads)
     rms_norm_staged_kernel(typename E::S* __restrict__ out, const typename E::S* __restrict__ x,
-                           typename E::S* __restrict__ res, const typename E::S* __restrict__ weight,
-                           int hidden, int64_t x_row_stride, float eps) {
+                           typename E::S* __restrict__ res, int64_t res_out,
+                           const typename E::S* __restrict__ weight, int hidden, RowMap x_rows, float eps) {
   using S = typename E::S;
   using P = Pack<S, VEC>;
   constexpr int kStagedPacks = kStageBytes / static_cast<int>(sizeof(P));
   __shared__ P staged[kStagedPacks];
   __shared__ float scratch[kMaxThreads / 64];
 
-  const int64_t row = blockIdx.x;
+  int64_t row, x_off;
+  x_rows.of_workgroup(&row, &x_off);
   const int packs = hidden / VEC;
   const int window = min(packs, kStagedPacks);
-  const P* xr = reinterpret_cast<const P*>(x + row * x_row_stride);
+  const P* xr = reinterpret_cast<const P*>(x + x_off);
   P* rr = HAS_RES ? reinterpret_cast<P*>(res + row * static_cast<int64_t>(hidden)) : nullptr;
+  P* rw = HAS_RES ? residual_out(rr, res_out) : nullptr;
   P* orow = reinterpret_cast<P*>(out + row * static_cast<int64_t>(hidden));
   const P* wr = reinterpret_cast<const P*>(weight);
 
@@ -340,7 +377,7 @@ __global__ void __launch_bounds__(kMaxThreads)
     }
     if (p < window) {
       staged[p] = v;
-      if constexpr (HAS_RES) rr[p] = v;
+      if constexpr (HAS_RES) rw[p] = v;
     }
   }
   const float rstd = inv_rms(block_sum(sum_sq, scratch), hidden, eps);
@@ -351,7 +388,7 @@ __global__ void __launch_bounds__(kMaxThreads)
       v = staged[p];
     } else {
       v = rounded_sum(p);
-      if constexpr (HAS_RES) rr[p] = v;
+      if constexpr (HAS_RES) rw[p] = v;
     }
     const P g = wr[p];
     P o;
@@ -372,13 +409,14 @@ constexpr int kRowsThreads = 256;
 template <typename E, int LANES, int NPACK, bool HAS_RES, bool ALIGNED>
 __global__ void __launch_bounds__(kRowsThreads)
     rms_norm_rows_kernel(typename E::S* __restrict__ out, const typename E::S* __restrict__ x,
-                         typename E::S* __restrict__ res, const typename E::S* __restrict__ weight, int rows, int hidden, int64_t x_row_stride, float eps) {
+                         typename E::S* __restrict__ res, int64_t res_out, const typename E::S* __restrict__ weight,
+                         int rows, int hidden, RowMap x_rows, float eps) {
   const int64_t r = static_cast<int64_t>(blockIdx.x) * (kRowsThreads / LANES) + threadIdx.x / LANES;
   const bool live = r < rows;
   const int64_t row = live ? r : rows - 1;
   norm_row<E, 16 / E::kBytes, NPACK, HAS_RES, ALIGNED>(
-      out + row * hidden, x + row * x_row_stride, HAS_RES ? res + row * hidden : nullptr, weight, hidden, eps,
-      threadIdx.x % LANES, LANES, live, [](float v) { return lanes_sum<LANES>(v); });
+      out + row * hidden, x + x_rows.x_of_row(row), HAS_RES ? res + row * hidden : nullptr,
+      res_out, weight, hidden, eps, threadIdx.x % LANES, LANES, live, [](float v) { return lanes_sum<LANES>(v); });
 }
 
 // Wide rows whose width or addresses are not multiples of 16 bytes: one
@@ -389,12 +427,14 @@ __global__ void __launch_bounds__(kRowsThreads)
 template <typename E, int NPACK, bool HAS_RES>
 __global__ void __launch_bounds__(kMaxThreads)
     rms_norm_ragged_kernel(typename E::S* __restrict__ out, const typename E::S* __restrict__ x,
-                           typename E::S* __restrict__ res, const typename E::S* __restrict__ weight, int hidden, int64_t x_row_stride, float eps) {
+                           typename E::S* __restrict__ res, int64_t res_out,
+                           const typename E::S* __restrict__ weight, int hidden, RowMap x_rows, float eps) {
   __shared__ float scratch[kMaxThreads / 64];
-  const int64_t row = blockIdx.x;
+  int64_t row, x_off;
+  x_rows.of_workgroup(&row, &x_off);
   norm_row<E, 16 / E::kBytes, NPACK, HAS_RES, false>(
-      out + row * hidden, x + row * x_row_stride, HAS_RES ? res + row * hidden : nullptr, weight, hidden, eps,
-      threadIdx.x, blockDim.x, true, [&](float v) { return block_sum(v, scratch); });
+      out + row * hidden, x + x_off, HAS_RES ? res + row * hidden : nullptr,
+      res_out, weight, hidden, eps, threadIdx.x, blockDim.x, true, [&](float v) { return block_sum(v, scratch); });
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -421,20 +461,22 @@ void with_packs(int npack, F&& f) {
 constexpr int kRowsMaxPacks = 64;
 
 template <typename E, bool HAS_RES>
-int launch_typed(void* out, const void* x, void* res, const void* w, int64_t rows, int hidden,
-                 int64_t x_row_stride, float eps, hipStream_t stream) {
+int launch_typed(void* out, const void* x, const void* res, void* res_out, const void* w, int64_t rows, int hidden,
+                 const RowMap& xm, float eps, hipStream_t stream) {
   using S = typename E::S;
   constexpr int VEC = 16 / E::kBytes;
   auto* o = static_cast<S*>(out);
   auto* xi = static_cast<const S*>(x);
-  auto* r = static_cast<S*>(res);
+  auto* r = static_cast<S*>(const_cast<void*>(res));  // read only, but for the in-place form
+  const int64_t rw = reinterpret_cast<intptr_t>(res_out) - reinterpret_cast<intptr_t>(res);
   auto* wi = static_cast<const S*>(w);
-  const bool aligned = hidden % VEC == 0 && x_row_stride % VEC == 0 && aligned16(out) && aligned16(x) &&
-                       aligned16(w) && (res == nullptr || aligned16(res));
+  const bool aligned = hidden % VEC == 0 && xm.row_stride % VEC == 0 && xm.group_stride % VEC == 0 &&
+                       aligned16(out) && aligned16(x) && aligned16(w) && aligned16(res) && aligned16(res_out);
   const int packs = static_cast<int>(cdiv(hidden, VEC));
-  const dim3 grid(static_cast<unsigned>(rows));
+  const auto gx = static_cast<unsigned>(xm.swapped ? rows / xm.inner : xm.inner);
+  const dim3 grid(gx, static_cast<unsigned>(rows / gx));
   if (hidden < VEC) {  // less than a pack: element by element
-    rms_norm_reg_kernel<E, 1, 1, HAS_RES><<<grid, 64, 0, stream>>>(o, xi, r, wi, hidden, x_row_stride, eps);
+    rms_norm_reg_kernel<E, 1, 1, HAS_RES><<<grid, 64, 0, stream>>>(o, xi, r, rw, wi, hidden, xm, eps);
     return check_launch("rms_norm kernel launch");
   }
   if (packs <= kRowsMaxPacks) {
@@ -443,10 +485,10 @@ int launch_typed(void* out, const void* x, void* res, const void* w, int64_t row
       const unsigned wgs = static_cast<unsigned>(cdiv(rows, kRowsThreads / L));
       if (aligned) {
         rms_norm_rows_kernel<E, L, NP, HAS_RES, true><<<wgs, kRowsThreads, 0, stream>>>(
-            o, xi, r, wi, static_cast<int>(rows), hidden, x_row_stride, eps);
+            o, xi, r, rw, wi, static_cast<int>(rows), hidden, xm, eps);
       } else {
         rms_norm_rows_kernel<E, L, NP, HAS_RES, false><<<wgs, kRowsThreads, 0, stream>>>(
-            o, xi, r, wi, static_cast<int>(rows), hidden, x_row_stride, eps);
+            o, xi, r, rw, wi, static_cast<int>(rows), hidden, xm, eps);
       }
     };
     if (packs <= 4) {
@@ -469,20 +511,20 @@ int launch_typed(void* out, const void* x, void* res, const void* w, int64_t row
   if (npack > (aligned ? 8 : 4)) {  // eight unaligned packs of x and the residual would spill
     if (aligned) {
       rms_norm_staged_kernel<E, VEC, HAS_RES>
-          <<<grid, kMaxThreads, 0, stream>>>(o, xi, r, wi, hidden, x_row_stride, eps);
+          <<<grid, kMaxThreads, 0, stream>>>(o, xi, r, rw, wi, hidden, xm, eps);
     } else {
       rms_norm_staged_kernel<E, 1, HAS_RES>
-          <<<grid, kMaxThreads, 0, stream>>>(o, xi, r, wi, hidden, x_row_stride, eps);
+          <<<grid, kMaxThreads, 0, stream>>>(o, xi, r, rw, wi, hidden, xm, eps);
     }
   } else {
     with_packs(npack, [&](auto np) {
       constexpr int NP = decltype(np)::value;
       if (aligned) {
         rms_norm_reg_kernel<E, VEC, NP, HAS_RES>
-            <<<grid, threads, 0, stream>>>(o, xi, r, wi, hidden, x_row_stride, eps);
+            <<<grid, threads, 0, stream>>>(o, xi, r, rw, wi, hidden, xm, eps);
       } else if constexpr (NP <= 4) {
         rms_norm_ragged_kernel<E, NP, HAS_RES>
-            <<<grid, threads, 0, stream>>>(o, xi, r, wi, hidden, x_row_stride, eps);
+            <<<grid, threads, 0, stream>>>(o, xi, r, rw, wi, hidden, xm, eps);
       }
     });
   }
@@ -490,38 +532,57 @@ int launch_typed(void* out, const void* x, void* res, const void* w, int64_t row
 }
 
 template <typename E>
-int launch_any(void* out, const void* x, void* res, const void* w, int64_t rows, int hidden, int64_t x_row_stride,
-               float eps, hipStream_t stream) {
-  return res ? launch_typed<E, true>(out, x, res, w, rows, hidden, x_row_stride, eps, stream)
-             : launch_typed<E, false>(out, x, res, w, rows, hidden, x_row_stride, eps, stream);
+int launch_any(void* out, const void* x, const void* res, void* res_out, const void* w, int64_t rows, int hidden,
+               const RowMap& xm, float eps, hipStream_t stream) {
+  return res ? launch_typed<E, true>(out, x, res, res_out, w, rows, hidden, xm, eps, stream)
+             : launch_typed<E, false>(out, x, nullptr, nullptr, w, rows, hidden, xm, eps, stream);
 }
 
 }  // namespace
 }  // namespace kl
 
-extern "C" int kl_rms_norm(kl_dtype dtype, void* out, const void* x, void* residual, const void* weight,
-                           int64_t rows, int64_t hidden, int64_t x_row_stride, float eps,
-                           kl_stream_t stream) {
+extern "C" int kl_rms_norm_grouped(kl_dtype dtype, void* out, const void* x, const void* residual, void* residual_out,
+                                   const void* weight, int64_t groups, int64_t rows_per_group, int64_t hidden,
+                                   int64_t x_group_stride, int64_t x_row_stride, float eps, kl_stream_t stream) {
   using namespace kl;
-  if (rows < 0 || hidden < 0) return fail(KL_ERR_INVALID_ARGUMENT, "rows and hidden must be >= 0");
-  if (rows == 0 || hidden == 0) return ok();
-  if (rows > 0x7fffffffLL) return fail(KL_ERR_UNSUPPORTED, "rows must be < 2^31");
+  if (groups < 0 || rows_per_group < 0 || hidden < 0) {
+    return fail(KL_ERR_INVALID_ARGUMENT, "rows and hidden must be >= 0");
+  }
+  if (groups == 0 || rows_per_group == 0 || hidden == 0) return ok();
+  if (groups > 0x7fffffffLL || rows_per_group > 0x7fffffffLL || groups * rows_per_group > 0x7fffffffLL) {
+    return fail(KL_ERR_UNSUPPORTED, "rows must be < 2^31");
+  }
   if (hidden > 0x7fffffffLL) return fail(KL_ERR_UNSUPPORTED, "hidden must be < 2^31");
   if (out == nullptr || x == nullptr || weight == nullptr) {
     return fail(KL_ERR_INVALID_ARGUMENT, "out, x and weight must be non-null");
   }
-  if (x_row_stride < hidden && rows > 1) {
-    return fail(KL_ERR_INVALID_ARGUMENT, "x_row_stride must be >= hidden");
+  if ((residual == nullptr) != (residual_out == nullptr)) {
+    return fail(KL_ERR_INVALID_ARGUMENT, "residual and residual_out go together");
+  }
+  if ((x_row_stride < hidden && rows_per_group > 1) || (x_group_stride < hidden && groups > 1)) {
+    return fail(KL_ERR_INVALID_ARGUMENT, "x_row_stride and x_group_stride must be >= hidden");
   }
   const auto s = reinterpret_cast<hipStream_t>(stream);
   const int h = static_cast<int>(hidden);
+  const int64_t rows = groups * rows_per_group;
+  // One row per group, or one group: a single stride. The grid's y is at most
+  // 65,535, which the smaller of two counts whose product is below 2^31 meets.
+  const RowMap xm = groups == 1           ? RowMap{rows, x_row_stride, 0, 0}
+                    : rows_per_group == 1 ? RowMap{rows, x_group_stride, 0, 0}
+                                          : RowMap{rows_per_group, x_row_stride, x_group_stride, groups > rows_per_group};
   switch (dtype) {
     case KL_DTYPE_F32:
-      return launch_any<F32>(out, x, residual, weight, rows, h, x_row_stride, eps, s);
+      return launch_any<F32>(out, x, residual, residual_out, weight, rows, h, xm, eps, s);
     case KL_DTYPE_F16:
-      return launch_any<F16>(out, x, residual, weight, rows, h, x_row_stride, eps, s);
+      return launch_any<F16>(out, x, residual, residual_out, weight, rows, h, xm, eps, s);
     case KL_DTYPE_BF16:
-      return launch_any<BF16>(out, x, residual, weight, rows, h, x_row_stride, eps, s);
+      return launch_any<BF16>(out, x, residual, residual_out, weight, rows, h, xm, eps, s);
   }
   return fail(KL_ERR_UNSUPPORTED, "dtype must be f32, f16 or bf16");
+}
+
+extern "C" int kl_rms_norm(kl_dtype dtype, void* out, const void* x, void* residual, const void* weight,
+                           int64_t rows, int64_t hidden, int64_t x_row_stride, float eps,
+                           kl_stream_t stream) {
+  return kl_rms_norm_grouped(dtype, out, x, residual, residual, weight, 1, rows, hidden, 0, x_row_stride, eps, stream);
 }

@@ -6,7 +6,8 @@
 //   fused_add_rms_norm(Tensor! out, Tensor x, Tensor! residual, Tensor weight, float eps) -> ()
 //   paged_decode_attention(Tensor! out, Tensor q, Tensor k_cache, Tensor v_cache,
 //                          Tensor block_table, Tensor seq_lens, float scale) -> ()
-// plus `fused_add_rmsnorm` (same schema as fused_add_rms_norm), the overload
+// plus `fused_add_rmsnorm` (same schema as fused_add_rms_norm),
+// `fused_add_rms_norm_new` (the new residual written to a tensor of its own), the overload
 // `paged_decode_attention.splits(..., int num_splits, int max_seq_len)` for
 // the split-KV controls of the reference's Triton wrapper
 // (kernel_lab/triton_kernels/paged_attention.py:176-211; 0 means "planner
@@ -81,57 +82,67 @@ void check_norm_args(const at::Tensor& out, const at::Tensor& x, const at::Tenso
   }
 }
 
-// x as `count` rows of its last dimension, row i at data + i * stride
-// elements. The kernels take one row stride, which the strides of x's
-// leading dimensions give when they nest (each steps over the next one's
-// span; size-1 dimensions are free). Otherwise, or when rows would overlap,
-// the rows are read from a contiguous copy: x is only read, so the result is
-// the same.
+// x as rows of its last dimension: `groups` groups of `inner` rows, row i of
+// group g at data + g * group_stride + i * row_stride elements. Leading
+// dimensions that nest (each steps over the next one's span; size-1 dimensions
+// are free) count as one, and the kernels address two. With more, or when rows
+// would overlap, the rows are read from a contiguous copy: x is only read, so
+// the result is the same.
 struct NormRows {
   at::Tensor data;  // x, or its contiguous copy
-  int64_t count;
-  int64_t stride;
+  int64_t groups, inner;
+  int64_t group_stride, row_stride;
 };
 
 NormRows norm_rows(const at::Tensor& x) {
   const int64_t hidden = x.size(-1);
   const int64_t count = hidden > 0 ? x.numel() / hidden : 0;
-  int64_t stride = hidden;  // a single row
-  bool nested = true;
-  int64_t inner_size = 0, inner_stride = 0;  // the next non-trivial dimension inward
+  if (count == 0) return {x, 0, 0, hidden, hidden};
+  int64_t size[2] = {1, 1}, stride[2] = {hidden, hidden};  // inner rows, groups
+  int level = -1;
   for (int64_t d = x.dim() - 2; d >= 0; --d) {
     if (x.size(d) == 1) continue;
-    if (inner_size == 0) {
-      stride = x.stride(d);  // the innermost leading dimension steps from row to row
-    } else if (x.stride(d) != inner_stride * inner_size) {
-      nested = false;
+    if (level >= 0 && x.stride(d) == stride[level] * size[level]) {
+      size[level] *= x.size(d);
+      continue;
     }
-    inner_size = x.size(d);
-    inner_stride = x.stride(d);
+    if (++level == 2) return {x.contiguous(), 1, count, 0, hidden};
+    size[level] = x.size(d);
+    stride[level] = x.stride(d);
   }
-  if (!nested || (count > 1 && stride < hidden)) return {x.contiguous(), count, hidden};
-  return {x, count, stride};
+  if (stride[0] < hidden || stride[1] < hidden) return {x.contiguous(), 1, count, 0, hidden};
+  return {x, size[1], size[0], stride[1], stride[0]};
 }
 
-void rms_norm_impl(at::Tensor& out, const at::Tensor& x, at::Tensor* residual, const at::Tensor& weight,
-                   double eps) {
+// residual null: the norm alone. residual_out: where the new residual goes
+// (residual itself for the in-place operators).
+void rms_norm_impl(at::Tensor& out, const at::Tensor& x, const at::Tensor* residual, at::Tensor* residual_out,
+                   const at::Tensor& weight, double eps) {
   check_norm_args(out, x, residual, weight);
+  if (residual_out != residual) check_norm_args(out, x, residual_out, weight);
   const NormRows rows = norm_rows(x);
-  if (rows.count == 0) return;
+  if (rows.groups == 0) return;
   const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
-  check_status(kl_rms_norm(to_kl_dtype(x.scalar_type()), out.data_ptr(), rows.data.data_ptr(),
-                           residual != nullptr ? residual->data_ptr() : nullptr, weight.data_ptr(), rows.count,
-                           x.size(-1), rows.stride, static_cast<float>(eps), current_stream(x.device())),
+  check_status(kl_rms_norm_grouped(to_kl_dtype(x.scalar_type()), out.data_ptr(), rows.data.data_ptr(),
+                                   residual != nullptr ? residual->data_ptr() : nullptr,
+                                   residual != nullptr ? residual_out->data_ptr() : nullptr, weight.data_ptr(),
+                                   rows.groups, rows.inner, x.size(-1), rows.group_stride, rows.row_stride,
+                                   static_cast<float>(eps), current_stream(x.device())),
                "rms_norm");
 }
 
 void rms_norm(at::Tensor& out, const at::Tensor& x, const at::Tensor& weight, double eps) {
-  rms_norm_impl(out, x, nullptr, weight, eps);
+  rms_norm_impl(out, x, nullptr, nullptr, weight, eps);
 }
 
 void fused_add_rms_norm(at::Tensor& out, const at::Tensor& x, at::Tensor& residual, const at::Tensor& weight,
                         double eps) {
-  rms_norm_impl(out, x, &residual, weight, eps);
+  rms_norm_impl(out, x, &residual, &residual, weight, eps);
+}
+
+void fused_add_rms_norm_new(at::Tensor& out, at::Tensor& residual_out, const at::Tensor& x, const at::Tensor& residual,
+                            const at::Tensor& weight, double eps) {
+  rms_norm_impl(out, x, &residual, &residual_out, weight, eps);
 }
 
 // Same checks as paged_decode_attention in the reference
@@ -311,6 +322,9 @@ void cascade_decode_attention(at::Tensor& out, const at::Tensor& q, const at::Te
 TORCH_LIBRARY(kernel_lab, m) {
   m.def("rms_norm(Tensor! out, Tensor x, Tensor weight, float eps) -> ()");
   m.def("fused_add_rms_norm(Tensor! out, Tensor x, Tensor! residual, Tensor weight, float eps) -> ()");
+  m.def(
+      "fused_add_rms_norm_new(Tensor! out, Tensor! residual_out, Tensor x, Tensor residual, Tensor weight, "
+      "float eps) -> ()");
   m.def("fused_add_rmsnorm(Tensor! out, Tensor x, Tensor! residual, Tensor weight, float eps) -> ()");
   m.def(
       "paged_decode_attention(Tensor! out, Tensor q, Tensor k_cache, Tensor v_cache, "
@@ -331,6 +345,7 @@ TORCH_LIBRARY(kernel_lab, m) {
 TORCH_LIBRARY_IMPL(kernel_lab, CUDA, m) {
   m.impl("rms_norm", &rms_norm);
   m.impl("fused_add_rms_norm", &fused_add_rms_norm);
+  m.impl("fused_add_rms_norm_new", &fused_add_rms_norm_new);
   m.impl("fused_add_rmsnorm", &fused_add_rms_norm);
   m.impl("paged_decode_attention", &paged_decode_attention);
   m.impl("paged_decode_attention.splits", &paged_decode_attention_splits);

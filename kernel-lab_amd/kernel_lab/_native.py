@@ -33,6 +33,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "kl_last_error": (ctypes.c_char_p, []),
     "kl_version": (_i32, []),
     "kl_rms_norm": (_i32, [_i32, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _f32, _vp]),
+    "kl_rms_norm_grouped": (_i32, [_i32, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _f32, _vp]),
     "kl_paged_decode_plan": (
         _i32,
         [_i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, ctypes.POINTER(_i32), ctypes.POINTER(_sz)],

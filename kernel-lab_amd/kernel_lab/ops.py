@@ -18,6 +18,7 @@ from __future__ import annotations
 import ctypes
 
 import torch
+from torch.autograd import forward_ad
 
 from kernel_lab import _native
 
@@ -49,6 +50,16 @@ def _rows_view(x: torch.Tensor) -> torch.Tensor:
     return x if x.stride(-1) == 1 else x.contiguous()
 
 
+def _carries_nothing(t: torch.Tensor) -> bool:
+    """Whether a clone of t would hold no more than its values: no autograd
+    history, forward-mode tangent or subclass."""
+    return (
+        type(t) in (torch.Tensor, torch.nn.Parameter)
+        and not (t.requires_grad and torch.is_grad_enabled())
+        and forward_ad._current_level < 0
+    )
+
+
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> torch.Tensor:
     """y = x / sqrt(mean(x^2) + eps) * weight over the last dimension."""
     _check_rms(x, weight, None)
@@ -71,8 +82,15 @@ def fused_add_rms_norm(
     _native.require_ops()
     x = _rows_view(x)
     out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    new_residual = residual.contiguous().clone()
-    torch.ops.kernel_lab.fused_add_rms_norm(out, x, new_residual, weight.contiguous(), eps)
+    residual = residual.contiguous()
+    if _carries_nothing(residual):
+        # The kernel reads the old residual and writes the new one: no clone
+        # (a launch of its own, and two more passes over the residual).
+        new_residual = torch.empty_like(residual)
+        torch.ops.kernel_lab.fused_add_rms_norm_new(out, new_residual, x, residual, weight.contiguous(), eps)
+    else:
+        new_residual = residual.clone()
+        torch.ops.kernel_lab.fused_add_rms_norm(out, x, new_residual, weight.contiguous(), eps)
     return out, new_residual
 
 
