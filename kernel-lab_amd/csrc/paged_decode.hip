@@ -217,9 +217,8 @@ __device__ __forceinline__ void unit_pages(const DecodeArgs& a, Unit& u) {
 
 // The unit of a uniform-split workgroup: b, kvh, hg and split from the
 // workgroup index (no memory access), then its length and page range.
-__device__ __forceinline__ Unit decode_unit_ids(const DecodeArgs& a) {
+__device__ __forceinline__ Unit decode_unit_ids(const DecodeArgs& a, int idx) {
   Unit u;
-  int idx = static_cast<int>(blockIdx.x);
   u.split = idx % a.num_splits;
   idx /= a.num_splits;
   u.hg = idx % a.head_groups;
@@ -230,7 +229,7 @@ __device__ __forceinline__ Unit decode_unit_ids(const DecodeArgs& a) {
 }
 
 __device__ __forceinline__ Unit decode_unit(const DecodeArgs& a) {
-  Unit u = decode_unit_ids(a);
+  Unit u = decode_unit_ids(a, static_cast<int>(blockIdx.x));
   unit_pages(a, u);
   return u;
 }
@@ -1364,7 +1363,7 @@ __global__ void __launch_bounds__((uniform_waves<E, D, NT>() * 64), (mfma_waves_
   // q and the first block-table window depend on the unit alone: they are
   // issued before the kernel waits for seq_lens, so the first K/V loads
   // follow one memory round trip after it instead of two.
-  Unit u = decode_unit_ids(a);
+  Unit u = decode_unit_ids(a, static_cast<int>(blockIdx.x));
   const int wave = wave_id();
   QFrag<NT, qk_chunks<E, D>()> q;
   load_q<E, D, NT>(a, u, q);
@@ -1373,7 +1372,7 @@ __global__ void __launch_bounds__((uniform_waves<E, D, NT>() * 64), (mfma_waves_
   unit_pages(a, u);
   if (u.page_begin >= u.page_end) {
     wait_vmcnt<0>();  // the window loads write this workgroup's LDS
-    if (u.split == 0 && u.seq_len <= 0 && (a.num_splits == 1 || a.arrivals != nullptr) && !a.force_partial) {
+    if (u.split == 0 && u.seq_len <= 0 && (a.num_splits == 1 || a.arrivals != nullptr)) {
       write_zero_heads<typename E::S, E>(a, u, D, threadIdx.x, blockDim.x);
     }
     return;  // a split past the end of its sequence has no work
@@ -1422,7 +1421,7 @@ __global__ void __launch_bounds__(2 * kThreads, (mfma_waves_per_eu<D, NT>()))
     // The other half's segment passes two workgroup barriers: pass them too.
     __syncthreads();
     __syncthreads();
-    if (u.split == 0 && u.seq_len <= 0 && (a.num_splits == 1 || a.arrivals != nullptr) && !a.force_partial) {
+    if (u.split == 0 && u.seq_len <= 0 && (a.num_splits == 1 || a.arrivals != nullptr)) {
       write_zero_heads<typename E::S, E>(a, u, D, threadIdx.x - half * kThreads, kThreads);
     }
     return;
@@ -2091,32 +2090,13 @@ __device__ __forceinline__ float wave_max(float v) {
   return fmaxf(fmaxf(lane_read(v, 0), lane_read(v, 16)), fmaxf(lane_read(v, 32), lane_read(v, 48)));
 }
 
-template <typename E, int kG, int POL>
-__device__ __forceinline__ void merge_partials(const float* lse, int64_t l_stride, const float* op,
-                                               int64_t o_stride, int n, int head_dim, typename E::S* out) {
+template <typename E, int kG, typename LoadO, typename LoadLse>
+__device__ __forceinline__ void merge_rows(int n, int head_dim, typename E::S* out, LoadO&& load_o, LoadLse&& load_lse) {
   const int lane = __lane_id();
   const int cpr = head_dim >> 2;      // 16-byte chunks per row (4 .. 64)
   const int rpl = 64 / cpr;           // rows per wave-wide load
   const int c = lane & (cpr - 1);
   const int r = lane / cpr;
-  // POL != 0: buffer loads with that cache policy (op and lse are
-  // wave-uniform, a unit's partials lie within 2 GiB of them).
-  const auto orsrc = make_rsrc(uniform_ptr(op));
-  const auto lrsrc = make_rsrc(uniform_ptr(lse));
-  auto load_o = [&](int w) -> f32x4 {
-    if constexpr (POL == 0) {
-      return *reinterpret_cast<const f32x4*>(op + w * o_stride + 4 * c);
-    } else {
-      return __builtin_bit_cast(f32x4, buffer_load16<POL>(orsrc, static_cast<uint32_t>((w * o_stride + 4 * c) * 4)));
-    }
-  };
-  auto load_lse = [&](int w) -> float {
-    if constexpr (POL == 0) {
-      return lse[w * l_stride];
-    } else {
-      return buffer_load_f32<POL>(lrsrc, static_cast<uint32_t>(w * l_stride * 4));
-    }
-  };
   f32x4 v[kG];
   float lw[kG];
   auto load_round = [&](int base) {
@@ -2156,6 +2136,33 @@ __device__ __forceinline__ void merge_partials(const float* lse, int64_t l_strid
 #pragma unroll
     for (int k = 0; k < 4; ++k) out[4 * c + k] = E::from_f32(acc[k] / den);
   }
+}
+
+template <typename E, int kG, int POL>
+__device__ __forceinline__ void merge_partials(const float* lse, int64_t l_stride, const float* op,
+                                               int64_t o_stride, int n, int head_dim, typename E::S* out) {
+  const int c = __lane_id() & ((head_dim >> 2) - 1);
+  // POL != 0: buffer loads with that cache policy (op and lse are
+  // wave-uniform, a unit's partials lie within 2 GiB of them).
+  const auto orsrc = make_rsrc(uniform_ptr(op));
+  const auto lrsrc = make_rsrc(uniform_ptr(lse));
+  merge_rows<E, kG>(
+      n, head_dim, out,
+      [&](int w) -> f32x4 {
+        if constexpr (POL == 0) {
+          return *reinterpret_cast<const f32x4*>(op + w * o_stride + 4 * c);
+        } else {
+          return __builtin_bit_cast(f32x4,
+                                    buffer_load16<POL>(orsrc, static_cast<uint32_t>((w * o_stride + 4 * c) * 4)));
+        }
+      },
+      [&](int w) -> float {
+        if constexpr (POL == 0) {
+          return lse[w * l_stride];
+        } else {
+          return buffer_load_f32<POL>(lrsrc, static_cast<uint32_t>(w * l_stride * 4));
+        }
+      });
 }
 
 // merge_partials split into a load phase and a finish phase, for merges whose
@@ -2286,7 +2293,57 @@ __global__ void __launch_bounds__(64) decode_merge_balanced_kernel(const DecodeA
 // the MFMA segment with all sequences' query heads of a KV head folded into
 // one group (q_fold), so each workgroup streams the prefix once for up to 32
 // query rows of many sequences; the suffix pass is the plain split decode.
-// Both write fp32 partials, and this kernel merges them by the LSE rule.
+// Both run in one launch and write fp32 partials, and a merge kernel combines
+// them by the LSE rule.
+
+// Both passes in one launch: the first pre_wgs workgroups take the prefix's
+// units, the rest the sequences' own, each as decode_mfma_kernel would. The
+// prefix pass waits on its chain of products (its K/V come from L2 after the
+// first head group) and the own pass on HBM, and the lengths of the own tokens
+// differ, so the two share the CUs better than they follow each other: a CU
+// holds two workgroups, and short ones make room for the next. What is left is
+// the two workgroups a CU runs one after the other, each a chain of blocks.
+// Measured, a launch per pass -> this, merge included (us): 32/8/128 fp16 B=64
+// prefix 4,096 own up to 1,024 55.1 -> 49.6, B=32 16,384 + 256 44.6 -> 39.1,
+// 64/8/128 bf16 B=16 16,384 + 1,024 47.9 -> 44.4, 32/8/128 B=4 2,000 + 300 18.5
+// -> 13.7. The own tokens first: 54.6; twice the prefix splits: 50.6; own
+// splits of 32 pages: 51.8. NTP, NTS: head tiles of the two passes.
+template <typename E, int D, int NT, int LDS>
+__device__ __forceinline__ void cascade_unit(const DecodeArgs& a, int idx, char (&lds)[LDS]) {
+  static_assert(MfmaLds<D, NT, kWaves, dma_staged<E, D, NT>()>::kBytes <= LDS);
+  fetch_args<dma_staged<E, D, NT>()>(a);
+  Unit u = decode_unit_ids(a, idx);
+  const int wave = wave_id();
+  QFrag<NT, qk_chunks<E, D>()> q;
+  load_q<E, D, NT>(a, u, q);
+  const int pb = u.split * a.pages_per_split;
+  prefetch_window<E, D, NT>(a, lds, u.b, pb, min(pb + a.pages_per_split, a.max_pages), wave);
+  unit_pages(a, u);
+  if (u.page_begin >= u.page_end) {
+    wait_vmcnt<0>();  // the window loads write this workgroup's LDS
+    return;
+  }
+  mfma_segment<E, E, D, NT>(a, lds, u, uniform_dest(a, u, D), wave, &q, true);
+}
+
+template <typename E, int D, int NTP, int NTS>
+constexpr int cascade_lds() {
+  constexpr int p = MfmaLds<D, NTP, kWaves, dma_staged<E, D, NTP>()>::kBytes;
+  constexpr int s = MfmaLds<D, NTS, kWaves, dma_staged<E, D, NTS>()>::kBytes;
+  return p > s ? p : s;
+}
+
+template <typename E, int D, int NTP, int NTS>
+__global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1)
+    cascade_decode_kernel(const DecodeArgs pre, const DecodeArgs suf, const int pre_wgs) {
+  __shared__ __attribute__((aligned(16))) char lds[cascade_lds<E, D, NTP, NTS>()];
+  const int idx = static_cast<int>(blockIdx.x);
+  if (idx < pre_wgs) {
+    cascade_unit<E, D, NTP>(pre, idx, lds);
+  } else {
+    cascade_unit<E, D, NTS>(suf, idx - pre_wgs, lds);
+  }
+}
 
 struct CascadeArgs {
   const float* p_o;          // prefix partials: virtual head kvh*(B*G) + b*G + g, p_splits each
@@ -2311,26 +2368,6 @@ __device__ __forceinline__ int active_splits(int len, int max_pages, int page_si
   return min(splits, (pages + pps - 1) / pps);
 }
 
-// Adds n partials (o_w at o + w*D, lse_w at lse[w]) to a running
-// sum_w 2^(lse_w - mx) o_w[d], loads issued eight partials at a time.
-__device__ __forceinline__ float merge_accumulate(const float* lse, const float* o, int n, int head_dim, int d,
-                                                  float mx) {
-  constexpr int U = 8;
-  float num = 0.0f;
-  for (int w0 = 0; w0 < n; w0 += U) {
-    float wt[U], v[U];
-#pragma unroll
-    for (int j = 0; j < U; ++j) {
-      const int w = min(w0 + j, n - 1);
-      wt[j] = lse[w];
-      v[j] = o[static_cast<int64_t>(w) * head_dim + d];
-    }
-#pragma unroll
-    for (int j = 0; j < U; ++j) num += (w0 + j < n ? exp2f(wt[j] - mx) : 0.0f) * v[j];
-  }
-  return num;
-}
-
 template <typename E>
 __global__ void __launch_bounds__(64) cascade_merge_kernel(const CascadeArgs c, int head_dim) {
   using S = typename E::S;
@@ -2352,18 +2389,15 @@ __global__ void __launch_bounds__(64) cascade_merge_kernel(const CascadeArgs c, 
   const float* po = c.p_o + vhead * c.p_splits * head_dim;
   const float* sl = c.s_lse + shead * c.s_splits;
   const float* so = c.s_o + shead * c.s_splits * head_dim;
-  float mx = -INFINITY;
-  for (int w = lane; w < np; w += 64) mx = fmaxf(mx, pl[w]);
-  for (int w = lane; w < ns; w += 64) mx = fmaxf(mx, sl[w]);
-  mx = wave_max(mx);
-  float den = 0.0f;
-  for (int w = lane; w < np; w += 64) den += exp2f(pl[w] - mx);
-  for (int w = lane; w < ns; w += 64) den += exp2f(sl[w] - mx);
-  den = wave_sum(den);
-  for (int d = lane; d < head_dim; d += 64) {
-    const float num = merge_accumulate(pl, po, np, head_dim, d, mx) + merge_accumulate(sl, so, ns, head_dim, d, mx);
-    out[d] = E::from_f32(num / den);
-  }
+  // The prefix's partials, then the sequence's own: one list of rows.
+  const int d = 4 * (lane & ((head_dim >> 2) - 1));
+  merge_rows<E, 8>(
+      np + ns, head_dim, out,
+      [&](int w) -> f32x4 {
+        const float* row = w < np ? po + static_cast<int64_t>(w) * head_dim : so + static_cast<int64_t>(w - np) * head_dim;
+        return *reinterpret_cast<const f32x4*>(row + d);
+      },
+      [&](int w) -> float { return w < np ? pl[w] : sl[w - np]; });
 }
 
 // -------------------------------------------------------------- host side
@@ -2799,7 +2833,7 @@ int make_plan(const Options& opt, kl_dtype dtype, int batch, int num_q_heads, in
   // Two adjacent KV heads per 8-wave workgroup when the pairs alone give
   // every CU a workgroup (one 8-wave workgroup per CU is the register budget)
   // and the 4-wave kernel fits two waves per SIMD (head_dim <= 128).
-  p->paired = mfma16 && whole_blocks && opt.pairing() && num_kv_heads % 2 == 0 && head_dim <= 128 && units * s / 2 >= cus;
+  p->paired = mfma16 && whole_blocks && !partials && opt.pairing() && num_kv_heads % 2 == 0 && head_dim <= 128 && units * s / 2 >= cus;
   if (s > 1 || partials) {
     const size_t rows = static_cast<size_t>(batch) * num_q_heads * s;
     p->o_bytes = align_up(rows * head_dim * sizeof(float));
@@ -3294,48 +3328,57 @@ int cascade_launch(const DecodeArgs& base, const CascadePlan& cp, const int32_t*
   const int batch = base.batch;
   const int num_q_heads = base.num_q_heads;
   const int group = base.group;
-  if (prefix_pages > 0) {
-    DecodeArgs a = base;
-    a.block_table = prefix_block_table;
-    a.seq_lens = prefix_len;
-    a.bt_stride = prefix_pages;
-    a.batch = 1;
-    a.group = batch * group;
-    a.num_q_heads = a.num_kv_heads * a.group;
-    a.max_pages = prefix_pages;
-    a.max_len = table_tokens(prefix_pages, a.page_size);
-    a.num_splits = cp.pre.num_splits;
-    a.pages_per_split = cp.pre.pages_per_split;
-    a.head_groups = cp.pre.head_groups;
-    a.heads_per_wg = cp.pre.heads_per_wg;
-    a.o_part = reinterpret_cast<float*>(ws);
-    a.lse_part = reinterpret_cast<float*>(ws + cp.pre.o_bytes);
-    a.paired = cp.pre.paired ? 1 : 0;
-    const int64_t wgs = static_cast<int64_t>(a.num_kv_heads) * a.head_groups * a.num_splits;
-    if (wgs > 0x7fffffffLL) return fail(KL_ERR_UNSUPPORTED, "too many workgroups");
-    int st = launch_uniform_mfma<E, E>(a, head_dim, static_cast<unsigned>(wgs), stream);
-    if (st != KL_OK) return st;
-    st = check_launch("cascade prefix pass launch");
-    if (st != KL_OK) return st;
-  }
+  DecodeArgs pre = base;
+  pre.block_table = prefix_block_table;
+  pre.seq_lens = prefix_len;
+  pre.bt_stride = prefix_pages;
+  pre.batch = 1;
+  pre.group = batch * group;
+  pre.num_q_heads = pre.num_kv_heads * pre.group;
+  pre.max_pages = prefix_pages;
+  pre.max_len = table_tokens(prefix_pages, base.page_size);
+  pre.num_splits = cp.pre.num_splits;
+  pre.pages_per_split = cp.pre.pages_per_split;
+  pre.head_groups = cp.pre.head_groups;
+  pre.heads_per_wg = cp.pre.heads_per_wg;
+  pre.o_part = reinterpret_cast<float*>(ws);
+  pre.lse_part = reinterpret_cast<float*>(ws + cp.pre.o_bytes);
   DecodeArgs a = base;
   a.block_table = block_table;
   a.seq_lens = seq_lens;
   a.bt_stride = bt_stride;
   a.max_pages = max_pages;
-  a.max_len = table_tokens(max_pages, a.page_size);
+  a.max_len = table_tokens(max_pages, base.page_size);
   a.num_splits = cp.suf.num_splits;
   a.pages_per_split = cp.suf.pages_per_split;
   a.head_groups = cp.suf.head_groups;
   a.heads_per_wg = cp.suf.heads_per_wg;
   a.o_part = reinterpret_cast<float*>(ws + cp.pre_bytes);
   a.lse_part = reinterpret_cast<float*>(ws + cp.pre_bytes + cp.suf.o_bytes);
-  a.paired = cp.suf.paired ? 1 : 0;
-  const int64_t wgs = static_cast<int64_t>(batch) * a.num_kv_heads * a.head_groups * a.num_splits;
+  const int64_t pre_wgs =
+      prefix_pages > 0 ? static_cast<int64_t>(pre.num_kv_heads) * pre.head_groups * pre.num_splits : 0;
+  const int64_t wgs = pre_wgs + static_cast<int64_t>(batch) * a.num_kv_heads * a.head_groups * a.num_splits;
   if (wgs > 0x7fffffffLL) return fail(KL_ERR_UNSUPPORTED, "too many workgroups");
-  int st = launch_uniform_mfma<E, E>(a, head_dim, static_cast<unsigned>(wgs), stream);
+  int st = dispatch_mfma(head_dim, a.heads_per_wg, [&](auto d, auto nts) -> int {
+    constexpr int D = decltype(d)::value, NTS = decltype(nts)::value;
+    auto launch = [&](auto ntp) {
+      cascade_decode_kernel<E, D, decltype(ntp)::value, NTS>
+          <<<static_cast<unsigned>(wgs), kThreads, 0, stream>>>(pre, a, static_cast<int>(pre_wgs));
+    };
+    // The prefix's folded group holds the sequences' own: at least their tiles.
+    if constexpr (D == 256) {
+      launch(IntC<1>{});
+    } else if constexpr (NTS == 2) {
+      launch(IntC<2>{});
+    } else if (pre.heads_per_wg > 16) {
+      launch(IntC<2>{});
+    } else {
+      launch(IntC<1>{});
+    }
+    return KL_OK;
+  });
   if (st != KL_OK) return st;
-  st = check_launch("cascade suffix pass launch");
+  st = check_launch("cascade decode kernel launch");
   if (st != KL_OK) return st;
 
   CascadeArgs c;

@@ -1,0 +1,41 @@
+"""Cascade decode's two passes in one launch: every pairing of their head tiles
+(one tile or two, i.e. up to 16 or more query heads per workgroup), the edges of
+blocks and splits on both sides, empty prefixes and empty own parts, and merges
+of more partials than one round loads."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from kernel_lab.kv_cache import random_cascade_problem
+from tests.test_hip_cascade import check, expected, run
+
+pytestmark = pytest.mark.gpu
+
+OWN = [0, 1, 15, 16, 17, 63, 64, 65, 130, 257]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("head_dim", [32, 64, 128, 256])
+@pytest.mark.parametrize(
+    ("hq", "hkv", "batch"),
+    [(8, 8, 2), (16, 4, 4), (16, 4, 10), (32, 1, 2), (20, 1, 10), (34, 2, 3)],
+    ids=["tiles 1/1 one head", "1/1 full tile", "2/1", "2/2", "2/2 ragged groups", "2/2 two heads"],
+)
+def test_head_tiles(gpu_ops, dtype, head_dim, hq, hkv, batch):
+    for prefix in (1, 257):
+        q, c = random_cascade_problem(prefix, OWN[:batch], hq, hkv, head_dim, 16, dtype=dtype, device="cuda", seed=prefix + hq)
+        check(run(gpu_ops, q, c), expected(q, c), dtype)
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+def test_many_partials(gpu_ops, head_dim):
+    """One unit: the prefix in 64 splits, the own tokens in up to 19."""
+    q, c = random_cascade_problem(17000, [5000, 0, 300], 4, 1, head_dim, 16, dtype=torch.bfloat16, device="cuda")
+    check(run(gpu_ops, q, c), expected(q, c), torch.bfloat16)
+
+
+def test_no_prefix_pages(gpu_ops):
+    q, c = random_cascade_problem(0, OWN, 32, 8, 128, 16, dtype=torch.float16, device="cuda")
+    check(run(gpu_ops, q, c), expected(q, c), torch.float16)
