@@ -199,6 +199,14 @@ constexpr bool kSmallPages = false;
 template <typename F>
 constexpr bool kSmallPages<SmallPages<F>> = true;
 
+// Cache format F on workgroups of eight waves per unit (balanced_waves).
+template <typename F>
+struct EightWaves : F {};
+template <typename KVF>
+constexpr bool kEightWaves = false;
+template <typename F>
+constexpr bool kEightWaves<EightWaves<F>> = true;
+
 struct Unit {
   int b, kvh, hg, split;
   int seq_len;          // clamped to max_pages * page_size
@@ -539,7 +547,7 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
   using S = typename E::S;
   using KS = typename KVF::S;          // cache storage type
   using M = Mfma<E>;
-  constexpr bool KV8 = std::is_same_v<KVF, Fp8E4M3>;
+  constexpr bool KV8 = KVF::kBytes == 1;
   constexpr bool FP32 = std::is_same_v<E, F32>;
   constexpr bool SP = kSmallPages<KVF>;
   constexpr int KB = KVF::kBytes;      // cache bytes per element
@@ -1726,15 +1734,35 @@ __device__ __forceinline__ Unit list_unit(const DecodeArgs& a, int hp, int ui, i
   return u;
 }
 
+// Waves per KV head of a balanced workgroup: four, or eight for FP8 caches at
+// head_dim 128 where the registers allow them. An FP8 block is half the bytes, so
+// four waves with a block each on its way leave a CU short of loads. Measured,
+// four -> eight (us, 128 head dims, FP8): 32/1 B=64 up to 8,192 tokens 31.2 ->
+// 27.0, B=16 18.1 -> 17.0, 16/4 B=32 up to 4,096 22.5 -> 19.3, 32/8 B=16 up to
+// 2,048 17.8 -> 16.7. With one head tile it pays only while the launch has no
+// more workgroups than CUs (wide_fp8): 8/1 B=300 up to 2,000 38.4 -> 44.6, 40/5
+// B=100 24.6 -> 26.4. Paired (16 waves) it spilled and lost: 32/8 B=64 of 4,096
+// 86.1 -> 90.4. Small pages in 16 bits lost too: 32/8 B=32 page 8 29.6 -> 32.4.
+template <typename KVF, int D, int NT, int PAIR>
+constexpr int balanced_waves() {
+  return kEightWaves<KVF> || (KVF::kBytes == 1 && D == 128 && NT == 2) ? 8 : kWaves;
+}
+template <typename KVF, int D, int NT, int PAIR>
+constexpr int balanced_waves_per_eu() {
+  const int waves = PAIR * balanced_waves<KVF, D, NT, PAIR>();
+  return std::max(mfma_waves_per_eu<D, NT>(), waves / 4);
+}
+
 // PAIR = 2 (num_kv_heads even): the work list's units are KV-head pairs (j,
 // head group); the workgroup has two halves of W waves that walk the same
 // segments, half h streaming KV head 2j + h with its own LDS (adjacent bytes
 // of every token row, as in decode_mfma_paired_kernel). Half h of segment
 // (list workgroup w, list unit u) owns partial slot (w + u) * 2 + h.
 template <typename E, typename KVF, int D, int NT, int PAIR>
-__global__ void __launch_bounds__(PAIR * kThreads, (mfma_waves_per_eu<D, NT>()))
+__global__ void __launch_bounds__((PAIR * balanced_waves<KVF, D, NT, PAIR>() * 64),
+                                  (balanced_waves_per_eu<KVF, D, NT, PAIR>()))
     decode_mfma_balanced_kernel(const DecodeArgs a) {
-  constexpr int W = kWaves;
+  constexpr int W = balanced_waves<KVF, D, NT, PAIR>();
   using Lds = MfmaLds<D, NT, W, dma_staged<KVF, D, NT>()>;
   __shared__ __attribute__((aligned(16))) char lds[PAIR * Lds::kBytes];
   __shared__ int s_last[PAIR];
@@ -1761,7 +1789,7 @@ __global__ void __launch_bounds__(PAIR * kThreads, (mfma_waves_per_eu<D, NT>()))
   QFrag<NT, qk_chunks<E, D>()> gq;
   if (a.even_start) {
     gu = list_unit<PAIR>(a, hp, w, half);
-    prefetch_window<KVF, D, NT>(a, lds + half * Lds::kBytes, gu.b, 0, a.max_pages, hw);
+    prefetch_window<KVF, D, NT, W>(a, lds + half * Lds::kBytes, gu.b, 0, a.max_pages, hw);
   }
   LenChunks lc;
   if (a.batch <= 64 * kScanChunks) lc = load_len_chunks(a);
@@ -2978,6 +3006,10 @@ int balanced_charge(int page_size, int head_dim, int kv_bytes, int paired, int h
       std::min<int64_t>(kMaxSegmentCharge, cdiv(kSegmentStartBytes + 2 * partial_bytes, page_bytes)));
 }
 
+// Whether an unpaired balanced launch of an FP8 cache with one head tile takes
+// eight waves per unit (balanced_waves).
+bool wide_fp8(const DecodeArgs& a) { return a.grid <= current_cu_count(); }
+
 template <typename E, typename KVF>
 int launch_balanced(DecodeArgs a, int head_dim, hipStream_t stream) {
   const unsigned grid = static_cast<unsigned>(a.grid);
@@ -2995,12 +3027,22 @@ int launch_balanced(DecodeArgs a, int head_dim, hipStream_t stream) {
         // One head tile and head_dim <= 128: beyond that the segment needs
         // more than the 256 registers per lane of an 8-wave workgroup.
         if constexpr (D <= 128 && NT == 1 && !kSmallPages<KVF>) {
-          decode_mfma_balanced_kernel<E, KVF, D, NT, 2><<<grid, 2 * kThreads, 0, stream>>>(a);
+          decode_mfma_balanced_kernel<E, KVF, D, NT, 2>
+              <<<grid, 2 * balanced_waves<KVF, D, NT, 2>() * 64, 0, stream>>>(a);
         } else {
           return fail(KL_ERR_UNSUPPORTED, "paired balanced decode needs head_dim <= 128 and <= 16 heads per workgroup");
         }
       } else {
-        decode_mfma_balanced_kernel<E, KVF, D, NT, 1><<<grid, kThreads, 0, stream>>>(a);
+        if constexpr (KVF::kBytes == 1 && D == 128 && NT == 1) {
+          if (wide_fp8(a)) {
+            using W8 = EightWaves<KVF>;
+            decode_mfma_balanced_kernel<E, W8, D, NT, 1>
+                <<<grid, balanced_waves<W8, D, NT, 1>() * 64, 0, stream>>>(a);
+            return KL_OK;
+          }
+        }
+        decode_mfma_balanced_kernel<E, KVF, D, NT, 1>
+            <<<grid, balanced_waves<KVF, D, NT, 1>() * 64, 0, stream>>>(a);
       }
       return KL_OK;
     } else {
