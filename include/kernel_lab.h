@@ -194,7 +194,7 @@ int kl_paged_decode_last_merge(void);
  * Re-reads the decode switches from the environment. The library reads them
  * once per process, at its first decode call; tests and A/B measurements
  * that change them afterwards call this. No counterpart in the reference.
- *   KL_DECODE_FORCE_VALU=1        fp16/bf16 decode on the VALU kernel
+ *   KL_DECODE_FORCE_VALU=1        decode on the VALU kernel
  *   KL_DECODE_PAIRED=0            no two-KV-head workgroups
  *   KL_DECODE_BALANCE_ALWAYS=1|0  full batches always / never balanced
  *   KL_DECODE_FUSED_MERGE=0       split sequences merged by a second launch

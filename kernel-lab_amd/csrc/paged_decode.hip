@@ -2466,7 +2466,7 @@ bool mfma_path(kl_dtype dtype, int head_dim) {
 // planned below. They are read from the environment once per process, at
 // the first call that needs them, and again by
 // kl_paged_decode_reload_options():
-//   KL_DECODE_FORCE_VALU=1        16-bit decode on the VALU kernel, so the
+//   KL_DECODE_FORCE_VALU=1        decode on the VALU kernel, so the
 //                                 benchmarks can time both paths on the same
 //                                 shapes (the FP8 and cascade entry points
 //                                 ignore it)
