@@ -2462,6 +2462,14 @@ bool mfma_path(kl_dtype dtype, int head_dim) {
   return head_dim == 32 && dtype != KL_DTYPE_F32;
 }
 
+// Whether a table of pages that do not hold whole blocks fits the SmallPages
+// arithmetic: its entries are loaded at 32-bit byte offsets from a buffer
+// resource of 2^31 - 1 bytes (an entry beyond reads as page 0), and a token
+// index is rounded up by as much as two blocks before it is clamped.
+bool small_pages_fit(int max_pages, int page_size) {
+  return max_pages <= 0x7fffffff / 4 && static_cast<int64_t>(max_pages) * page_size <= 0x7fffffff - 2 * kBlock;
+}
+
 // Switches for A/B measurements and tests; unset, the library behaves as
 // planned below. They are read from the environment once per process, at
 // the first call that needs them, and again by
@@ -2716,14 +2724,13 @@ int make_plan(const Options& opt, kl_dtype dtype, int batch, int num_q_heads, in
   // Pages that do not hold whole blocks: a split or a workgroup's range is
   // counted in pages of one block when the planner chooses it, so the rules
   // below see the lengths they were measured at, and in the table's own pages
-  // when the caller gives the split count, as the original counts them. The
-  // few tables whose length in blocks passes an int keep the VALU kernel.
-  const int64_t blocks = cdiv(static_cast<int64_t>(max_pages) * page_size, kBlock);
-  const bool mfma = use_mfma && mfma_path(dtype, head_dim) && (whole_blocks || blocks <= 0x7fffffff);
+  // when the caller gives the split count, as the original counts them. Tables
+  // beyond small_pages_fit keep the VALU kernel.
+  const bool mfma = use_mfma && mfma_path(dtype, head_dim) && (whole_blocks || small_pages_fit(max_pages, page_size));
   p->mfma = mfma;
   if (mfma && !whole_blocks && num_splits <= 0) {
+    max_pages = static_cast<int>(cdiv(static_cast<int64_t>(max_pages) * page_size, kBlock));
     page_size = kBlock;
-    max_pages = static_cast<int>(blocks);
   }
   p->page_size = page_size;
   p->max_pages = max_pages;

@@ -252,6 +252,21 @@ def test_out_of_range_dtypes_are_rejected(dtype):
                                          None) == 2
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize(
+    ("page", "max_pages", "mfma"),
+    [(1, 536870911, True), (1, 536870912, False), (2, 536870911, True), (2, 536870912, False), (3, 536870912, False),
+     (5, 429496723, True), (5, 429496724, False), (24, 89478483, True), (24, 89478484, False), (16, 536870912, True)],
+)
+def test_small_page_tables_stay_within_the_index_arithmetic(dtype, page, max_pages, mfma):
+    """Small-page tables whose columns pass 2^31 bytes, or whose tokens come
+    within two blocks of 2^31, take the VALU kernel, which addresses with 64
+    bits. Its workgroups hold 8 query heads and the MFMA ones 16, so 8
+    sequences of one 16-head group are cut into 16 or 32 splits."""
+    splits, _ = ops.plan_decode(dtype, 8, 16, 1, 64, page, max_pages, 0, 256)
+    assert splits == (32 if mfma else 16)
+
+
 def test_planner_rejects_bad_shapes():
     with pytest.raises(ValueError, match="multiple"):
         ops.plan_decode(torch.float16, 2, 3, 2, 128, 16, 4)
