@@ -199,6 +199,18 @@ constexpr bool kSmallPages = false;
 template <typename F>
 constexpr bool kSmallPages<SmallPages<F>> = true;
 
+// Whether the softmax weights keep fp32's precision up to the P V products, as
+// the VALU kernel's do: fp32, and small pages, which are 16-bit caches whose
+// weights go in as three bf16 parts or two fp16 ones (2^-24 of a weight). A
+// weight of bf16 under 2^-120 of the largest, of fp16 under 2^-33, counts as 0.
+// Measured (us, bf16, two parts -> three): 32/8/128 page 8 B=32 up to 2,048
+// tokens 28.7 -> 29.3, 32/8/64 24.2 -> 25.7, 32/1/128 up to 8,192 24.1 -> 26.7;
+// with fp32 MFMAs throughout 36.5, 32.0 and 33.2.
+template <typename E, typename KVF>
+constexpr bool fp32_weights() {
+  return std::is_same_v<E, F32> || kSmallPages<KVF>;
+}
+
 // Cache format F on workgroups of eight waves per unit (balanced_waves).
 template <typename F>
 struct EightWaves : F {};
@@ -550,6 +562,13 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
   constexpr bool KV8 = KVF::kBytes == 1;
   constexpr bool FP32 = std::is_same_v<E, F32>;
   constexpr bool SP = kSmallPages<KVF>;
+  constexpr bool P32 = fp32_weights<E, KVF>();
+  // log2 of the weight that moves the reference max, and of the weight the
+  // score that moved it then has. P32: bf16 weights stay at most 1, so that a
+  // large value's product does not overflow; fp16's values are small and the
+  // parts of a small weight subnormal, so its weights are large.
+  constexpr float kMostLog = !P32 ? kRescaleSlack : std::is_same_v<E, F16> ? 15.0f : 0.0f;
+  constexpr float kTopLog = !P32 || FP32 ? 0.0f : kMostLog - 6.0f;
   constexpr int KB = KVF::kBytes;      // cache bytes per element
   constexpr int KC = qk_chunks<E, D>();  // QK k-chunks
   constexpr int DT = D / 16;           // PV output tiles along head_dim
@@ -588,13 +607,16 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
 
   float m[NT], l[NT];
   f32x4 acc[NT][DT];
+  auto start_sums = [&] {
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    m[t] = -INFINITY;
-    l[t] = 0.0f;
+    for (int t = 0; t < NT; ++t) {
+      m[t] = -INFINITY;
+      l[t] = 0.0f;
 #pragma unroll
-    for (int d = 0; d < DT; ++d) acc[t][d] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  }
+      for (int d = 0; d < DT; ++d) acc[t][d] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+  };
+  start_sums();
 
   const KS* kc = static_cast<const KS*>(a.k);
   const KS* vc = static_cast<const KS*>(a.v);
@@ -812,12 +834,14 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
   // operand of S = K Q^T: lane holds token `row`, dims 32c + 8grp .. +7),
   // a stage_v(nvalid) step run before the V tiles are read, and v_tile(dt),
   // which reads V^T tile dt (lane holds V[token 4grp + j][dim 16dt + row]).
-  auto compute_block = [&](int i, const u32x4 (&ka)[KC], auto&& stage_v, auto&& v_tile) {
+  auto compute_block = [&](int i, const u32x4 (&ka)[KC], auto&& stage_v, auto&& v_tile, auto exact) {
     const int nvalid = valid_of(i);
 
     // Scores: lane holds S[token 4grp + i][head row] for tile t.
-    u32x2 pf[NT], pl[NT];
-    f32x4 p32[NT];  // fp32: the weights as they are
+    constexpr bool kExact = decltype(exact)::value;
+    constexpr bool kThirdPart = P32 && std::is_same_v<E, BF16>;
+    u32x2 pf[NT], pl[NT], pr[NT];  // the weights' 16-bit parts: two, or three
+    f32x4 p32[NT];                 // kExact: the weights as they are
     float alpha[NT];
     bool grew = false;
 #pragma unroll
@@ -862,23 +886,35 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
       // normaliser and the log-sum-exp all refer to it. A real block's token
       // 0 is valid, so mx is finite; the first block always moves m off
       // -inf; a padding slot has mx = -inf and leaves m as it is.
-      const float m_new = mx > m[t] + (FP32 ? 0.0f : kRescaleSlack) ? mx : m[t];
+      const float m_new = mx > m[t] + kMostLog ? mx - kTopLog : m[t];
       grew |= m_new > m[t];
-      alpha[t] = __builtin_amdgcn_exp2f(m[t] - m_new);
       float p[4];
+      if constexpr (P32) {
+        alpha[t] = __builtin_amdgcn_exp2f(m[t] - m_new);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) p[j] = __builtin_amdgcn_exp2f(FP32 ? fmaf(s[j], qk_scale, -m_new) : sc[j] - m_new);
-      if (FP32 && nvalid < kBlock) {
+        for (int j = 0; j < 4; ++j) p[j] = __builtin_amdgcn_exp2f(fmaf(s[j], qk_scale, -m_new));
+      } else {
+        alpha[t] = __builtin_amdgcn_exp2f(m[t] - m_new);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) p[j] = __builtin_amdgcn_exp2f(sc[j] - m_new);
+      }
+      if (P32 && nvalid < kBlock) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) p[j] = (4 * grp + j < nvalid) ? p[j] : 0.0f;
       }
       l[t] = l[t] * alpha[t] + ((p[0] + p[1]) + (p[2] + p[3]));
       m[t] = m_new;
-      if constexpr (FP32) {
+      if constexpr (kExact) {
         p32[t] = f32x4{p[0], p[1], p[2], p[3]};
       } else {
         pf[t] = u32x2{pack2<E>(p[0], p[1]), pack2<E>(p[2], p[3])};
         pl[t] = u32x2{pack2_residual<E>(p[0], p[1], pf[t][0]), pack2_residual<E>(p[2], p[3], pf[t][1])};
+        if constexpr (kThirdPart) {
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            pr[t][h] = pack2_residual<E>(p[2 * h] - lo_f32<E>(pf[t][h]), p[2 * h + 1] - hi_f32<E>(pf[t][h]), pl[t][h]);
+          }
+        }
       }
     }
     // Rescale the outputs only when some head's running max moved (alpha < 1).
@@ -896,8 +932,9 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
       const auto va = v_tile(dt);
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
+        // fp32 products, k step j: token 4grp + j, whose weight p[j] this lane
+        // holds as B.
         if constexpr (FP32) {
-          // k step j: token 4grp + j, whose weight p[j] this lane holds as B.
           // The block's products are summed on their own, in two halves, so
           // the long running sum takes one rounding per block.
           const f32x4 vv = __builtin_bit_cast(f32x4, va);
@@ -908,8 +945,18 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
             step[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[j], p32[t][j], before, 0, 0, 0);
           }
           acc[t][dt] += step[2] + step[3];
+        } else if constexpr (kExact) {
+          const float vv[4] = {lo_f32<E>(va[0]), hi_f32<E>(va[0]), lo_f32<E>(va[1]), hi_f32<E>(va[1])};
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            acc[t][dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[j], p32[t][j], acc[t][dt], 0, 0, 0);
+          }
         } else {
           acc[t][dt] = pv_split<E>(va, pf[t], pl[t], acc[t][dt]);
+          // The third part by the same instruction: the compiler lets a
+          // 16x16x16 product follow a 16x16x32 one on its accumulator sooner
+          // than the hardware does (outputs lost the first one's).
+          if constexpr (kThirdPart) acc[t][dt] = pv_split<E>(va, pr[t], u32x2{0, 0}, acc[t][dt]);
         }
       }
     }
@@ -917,7 +964,7 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
 
   // Register pipeline: block i's K and V arrive in registers (kf, vf) and are
   // re-laid out through this wave's LDS tile.
-  auto process_block = [&](auto i, const u32x4 (&kf)[NL], const u32x4 (&vf)[NL]) {
+  auto process_block = [&](auto i, const u32x4 (&kf)[NL], const u32x4 (&vf)[NL], auto exact) {
     // Stage K (its rows past seq_len only feed scores replaced by -inf).
 #pragma unroll
     for (int c = 0; c < NL; ++c) stage16(kstage + load_tok(c) * KROW + load_dim(c), kf[c]);
@@ -934,7 +981,7 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
             stage16(stage + tok * VROW + load_dim(c), tok < nvalid ? vf[c] : u32x4{0, 0, 0, 0});
           }
         },
-        [&](int dt) { return lds_read_tr16(tr_src + 16 * dt); });
+        [&](int dt) { return lds_read_tr16(tr_src + 16 * dt); }, exact);
   };
 
   // LDS pipeline: block i's K and V load straight into its LDS slot (rows
@@ -947,7 +994,8 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
     u32x4 ka[KC];
 #pragma unroll
     for (int c = 0; c < KC; ++c) ka[c] = *reinterpret_cast<const u32x4*>(ks + (k_rd ^ (c << 5)));
-    compute_block(i, ka, [&](int) { wait_v(); }, [&](int dt) { return lds_read_tr16(vs + (v_rd ^ (dt << 4))); });
+    compute_block(i, ka, [&](int) { wait_v(); }, [&](int dt) { return lds_read_tr16(vs + (v_rd ^ (dt << 4))); },
+                  std::false_type{});
   };
 
   if constexpr (kDma) {
@@ -1042,7 +1090,8 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
             [&](int dt) {
               const int h = dt & ~3, e = dt & 3;
               return u32x4{vf[h][e], vf[h + 1][e], vf[h + 2][e], vf[h + 3][e]};
-            });
+            },
+            std::true_type{});
         load_half(vc, src, vf, more);
       }
     }
@@ -1080,7 +1129,26 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
         const auto next = block_src(j, pg[slot]);
         pg[slot] = table_load(min(i + 2 * NS - 1, nblk - 1));
         load_block(next, kb[slot], vb[slot], i + NS - 1 < nblk);
-        process_block(i, kb[s], vb[s]);
+        process_block(i, kb[s], vb[s], std::false_type{});
+      }
+    }
+    if constexpr (P32) {
+      // A part of a weight that is 0, or of the other sign, makes an infinite
+      // V value NaN where the weight itself would not: a wave whose outputs
+      // are not numbers goes over its blocks again with the weights whole.
+      f32x4 total = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) total += acc[t][dt];
+      }
+      const float any = (total[0] + total[1]) + (total[2] + total[3]);
+      if (__any(any != any)) {
+        start_sums();
+        for (int i = 0; i < nblk; ++i) {
+          load_block(first_src(i), kb[0], vb[0], true);
+          process_block(i, kb[0], vb[0], std::true_type{});
+        }
       }
     }
   }
@@ -1154,7 +1222,7 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
       for (int w = 1; w < W; ++w) num += lds_acc[(w * NT * DT + t * DT + dt) * 64 + lane] * cw[w];
       float o[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] = FP32 ? num[i] / denom : num[i] * inv;
+      for (int i = 0; i < 4; ++i) o[i] = P32 ? num[i] / denom : num[i] * inv;
       if (!valid) continue;
       const int d = FP32 ? 16 * (dt & ~3) + 16 * grp + 4 * (dt & 3) : 16 * dt + 4 * grp;
       if (dst.final) {

@@ -66,3 +66,21 @@ def test_small_pages_empty_sequences(gpu_ops):
     for splits in (None, 2, -1):
         out = gpu_ops.paged_decode_attention(q, kv.k_cache, kv.v_cache, kv.block_table, kv.seq_lens, num_splits=splits)
         assert (out[1] == 0).all() and torch.isfinite(out).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("splits", [None, 3])
+def test_small_pages_infinite_values(gpu_ops, dtype, splits):
+    """An infinite value with a positive weight gives an infinite output in its
+    head dim and leaves the others alone."""
+    q, kv, _, _ = random_decode_problem([700, 40, 5], 8, 2, 128, 8, dtype=dtype, device="cuda")
+    for b, tok in ((0, 333), (1, 39), (2, 0)):
+        page = int(kv.block_table[b, tok // 8])
+        kv.v_cache[page, tok % 8, 0, 7] = float("inf")
+        kv.v_cache[page, tok % 8, 1, 100] = -float("inf")
+    out = gpu_ops.paged_decode_attention(q, kv.k_cache, kv.v_cache, kv.block_table, kv.seq_lens, num_splits=splits).cpu()
+    assert (out[:, :4, 7] == float("inf")).all() and (out[:, 4:, 100] == -float("inf")).all()
+    want = ref.paged_decode_attention(q.cpu().float(), kv.k_cache.cpu(), kv.v_cache.cpu(), kv.block_table.cpu(), kv.seq_lens.cpu())
+    finite = torch.isfinite(want)
+    assert int((~finite).sum()) == 3 * 8
+    decode_parity(out.masked_fill(~finite, 0), want.masked_fill(~finite, 0), dtype)
