@@ -890,9 +890,12 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
       grew |= m_new > m[t];
       float p[4];
       if constexpr (P32) {
-        alpha[t] = __builtin_amdgcn_exp2f(m[t] - m_new);
+        // Scores of -inf alone leave the reference at -inf: any finite one
+        // gives them 0.
+        const float m_ref = m_new == -INFINITY ? 0.0f : m_new;
+        alpha[t] = __builtin_amdgcn_exp2f(m[t] - m_ref);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) p[j] = __builtin_amdgcn_exp2f(fmaf(s[j], qk_scale, -m_new));
+        for (int j = 0; j < 4; ++j) p[j] = __builtin_amdgcn_exp2f(fmaf(s[j], qk_scale, -m_ref));
       } else {
         alpha[t] = __builtin_amdgcn_exp2f(m[t] - m_new);
 #pragma unroll
@@ -1211,6 +1214,9 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
       denom += lw[w] * cw[w];
     }
     const float inv = out_scale / denom;
+    // P32: a partial of nothing but -inf scores weighs 2^-inf in the merge, so
+    // it must be a number.
+    const bool no_weight = P32 && !dst.final && denom == 0.0f;
     const int hl = h0 + 16 * t + row;
     const bool valid = hl < a.group;
     const int64_t head = q_row(a, u, valid ? hl : 0);
@@ -1222,7 +1228,7 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
       for (int w = 1; w < W; ++w) num += lds_acc[(w * NT * DT + t * DT + dt) * 64 + lane] * cw[w];
       float o[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] = P32 ? num[i] / denom : num[i] * inv;
+      for (int i = 0; i < 4; ++i) o[i] = !P32 ? num[i] * inv : no_weight ? 0.0f : num[i] / denom;
       if (!valid) continue;
       const int d = FP32 ? 16 * (dt & ~3) + 16 * grp + 4 * (dt & 3) : 16 * dt + 4 * grp;
       if (dst.final) {
