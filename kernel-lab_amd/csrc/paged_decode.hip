@@ -891,11 +891,23 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
       float p[4];
       if constexpr (P32) {
         // Scores of -inf alone leave the reference at -inf: any finite one
-        // gives them 0.
+        // gives them 0. The hardware exponential flushes results below 2^-126:
+        // where the weights stay whole, a wave with one such takes exp2f,
+        // which is the same elsewhere.
         const float m_ref = m_new == -INFINITY ? 0.0f : m_new;
-        alpha[t] = __builtin_amdgcn_exp2f(m[t] - m_ref);
+        const float a_log = m[t] - m_ref;
+        float p_log[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) p[j] = __builtin_amdgcn_exp2f(fmaf(s[j], qk_scale, -m_ref));
+        for (int j = 0; j < 4; ++j) p_log[j] = fmaf(s[j], qk_scale, -m_ref);
+        if (kExact && __any(fminf(fminf(fminf(p_log[0], p_log[1]), fminf(p_log[2], p_log[3])), a_log) < -126.0f)) {
+          alpha[t] = exp2f(a_log);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) p[j] = exp2f(p_log[j]);
+        } else {
+          alpha[t] = __builtin_amdgcn_exp2f(a_log);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) p[j] = __builtin_amdgcn_exp2f(p_log[j]);
+        }
       } else {
         alpha[t] = __builtin_amdgcn_exp2f(m[t] - m_new);
 #pragma unroll
@@ -1204,13 +1216,14 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
       lw[w] = lds_ml[((w * NT + t) * 16 + row) * 2 + 1];
       mmax = fmaxf(mmax, mw[w]);
     }
-    // Weights 2^(m_w - max) lie in [0, 1]: the hardware exponential suffices
-    // (one whose result is denormal contributes nothing visible).
+    // Weights 2^(m_w - max) lie in [0, 1]: for 16-bit weights the hardware
+    // exponential suffices (one whose result is denormal contributes nothing
+    // visible).
     float cw[W];
     float denom = 0.0f;
 #pragma unroll
     for (int w = 0; w < W; ++w) {
-      cw[w] = mw[w] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mw[w] - mmax);
+      cw[w] = mw[w] == -INFINITY ? 0.0f : P32 ? exp2f(mw[w] - mmax) : __builtin_amdgcn_exp2f(mw[w] - mmax);
       denom += lw[w] * cw[w];
     }
     const float inv = out_scale / denom;
@@ -1250,7 +1263,7 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
     if (valid && !dst.final && grp == 0 && (t * DT) % W == wave) {
       buffer_store_f32<kCachePolicyDevice>(make_rsrc(uniform_ptr(dst.lse)),
                                            static_cast<uint32_t>((16 * t + row) * dst.lse_head_stride * 4),
-                                           mmax + __builtin_amdgcn_logf(denom));
+                                           mmax + (P32 ? log2f(denom) : __builtin_amdgcn_logf(denom)));
     }
   }
 }

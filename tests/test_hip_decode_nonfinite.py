@@ -1,7 +1,10 @@
-"""Decode where scores are -inf, on the paths with fp32 weights (fp32 caches and
-small pages), against the CPU oracle."""
+"""Decode at the edges of the number range, on the paths with fp32 weights (fp32
+caches and small pages): scores of -inf against the CPU oracle, and weights
+below the normal range."""
 
 from __future__ import annotations
+
+import math
 
 import pytest
 import torch
@@ -26,3 +29,24 @@ def test_blocks_of_minus_infinity(gpu_ops, dtype, page, splits, masked):
     out = gpu_ops.paged_decode_attention(q, kv.k_cache, kv.v_cache, kv.block_table, kv.seq_lens, num_splits=splits)
     want = ref.paged_decode_attention(q.cpu().float(), kv.k_cache.cpu(), kv.v_cache.cpu(), kv.block_table.cpu(), kv.seq_lens.cpu())
     decode_parity(out, want, dtype, f"{masked}")
+
+
+@pytest.mark.parametrize("page", [16, 8])
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("far", [17, 255])
+def test_weights_below_the_normal_range(gpu_ops, page, splits, far):
+    """One value of 1e38 at a weight of e^-90 (2^-130, a subnormal: 19 bits)
+    among zeros. 1e-4 covers the subnormal's rounding (2^-20), its split's
+    normaliser and the exponent's (90 / ln 2 at 2^-24 of itself)."""
+    q, kv, _, _ = random_decode_problem([256], 4, 1, 64, page, dtype=torch.float32, device="cuda")
+    q.zero_()
+    q[..., 0] = 8.0
+    kv.k_cache.zero_()
+    kv.v_cache.zero_()
+    kv.k_cache[..., 0] = 90.0
+    at = (int(kv.block_table[0, far // page]), far % page, 0)
+    kv.k_cache[at][0] = 0.0
+    kv.v_cache[at] = 1e38
+    out = gpu_ops.paged_decode_attention(q, kv.k_cache, kv.v_cache, kv.block_table, kv.seq_lens, num_splits=splits)
+    want = math.exp(-90.0) / 255 * 1e38
+    assert (out.cpu().double() - want).abs().max() <= 1e-4 * want
