@@ -140,13 +140,6 @@ struct DecodeArgs {
   uint32_t bpp_magic;
   int bpp_shift;
   int max_pages;
-  int max_len;          // longest length a sequence may have: seq_lens beyond it count as it
-  // Caches whose pages do not hold whole blocks (SmallPages): the block table's
-  // page size, and the division by it. page_size and max_pages are then the
-  // schedule's, which need not be the table's.
-  int table_page;
-  uint32_t table_magic;
-  int table_shift;
   int num_splits;
   int pages_per_split;
   int head_groups;      // workgroups per (sequence, KV head, split) along the group
@@ -173,7 +166,20 @@ struct DecodeArgs {
   // Fused merge: this call's arrival counters, one per unit, zero on entry
   // and left zero (null: a merge kernel combines the partials).
   uint32_t* arrivals;
+  // Caches whose pages do not hold whole blocks (SmallPages): the block table's
+  // page size, the division by it, and the tokens the table holds. page_size
+  // and max_pages are then the schedule's, which need not be the table's.
+  int table_page;
+  uint32_t table_magic;
+  int table_shift;
+  int table_tokens;
 };
+
+// seq_lens as the kernels count it: at most what max_pages pages hold.
+__device__ __forceinline__ int clamped_len(const DecodeArgs& a, int raw) {
+  const int64_t cap = static_cast<int64_t>(a.max_pages) * a.page_size;
+  return static_cast<int>(raw < cap ? raw : cap);
+}
 
 // Block index -> page index (n >= 0, wave-uniform or per lane).
 __device__ __forceinline__ int block_page(const DecodeArgs& a, int n) {
@@ -229,7 +235,7 @@ struct Unit {
 // split are set.
 __device__ __forceinline__ void unit_pages(const DecodeArgs& a, Unit& u) {
   const int raw = as_constant(a.seq_lens)[u.b];
-  u.seq_len = min(raw, a.max_len);
+  u.seq_len = clamped_len(a, raw);
   const int num_pages = u.seq_len > 0 ? (u.seq_len + a.page_size - 1) / a.page_size : 0;
   u.page_begin = u.split * a.pages_per_split;
   u.page_end = min(u.page_begin + a.pages_per_split, num_pages);
@@ -453,15 +459,16 @@ struct Dest {
 // such load in turn; the uniform decode kernel's prologue showed three
 // dependent argument round trips before its first q load. Naming the fields
 // the kernels read as inputs of an empty asm statement has them loaded before
-// it, with one wait. kWindow: the kernel loads block-table windows, the only
-// readers of max_pages.
-template <bool kWindow>
+// it, with one wait.
+template <bool kSmall = false>
 __device__ __forceinline__ void fetch_args(const DecodeArgs& a) {
-  if constexpr (kWindow) asm volatile("" ::"s"(a.max_pages));
+  if constexpr (kSmall) {
+    asm volatile("" ::"s"(a.table_page), "s"(a.table_magic), "s"(a.table_shift), "s"(a.table_tokens));
+  }
   asm volatile("" ::"s"(a.q), "s"(a.k), "s"(a.v), "s"(a.out), "s"(a.block_table), "s"(a.seq_lens), "s"(a.o_part),
                "s"(a.lse_part), "s"(a.bt_stride), "s"(a.page_stride), "s"(a.arrivals));
   asm volatile("" ::"s"(a.token_stride), "s"(a.batch), "s"(a.num_q_heads), "s"(a.num_kv_heads), "s"(a.group),
-               "s"(a.page_size), "s"(a.bpp_magic), "s"(a.bpp_shift), "s"(a.max_len), "s"(a.num_splits),
+               "s"(a.page_size), "s"(a.bpp_magic), "s"(a.bpp_shift), "s"(a.max_pages), "s"(a.num_splits),
                "s"(a.pages_per_split), "s"(a.head_groups), "s"(a.heads_per_wg), "s"(a.grid), "s"(a.even_start),
                "s"(a.seg_charge), "s"(a.scale_log2),
                "s"(a.q_fold), "s"(a.q_heads), "s"(a.force_partial));
@@ -632,8 +639,9 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
   const int blk_begin = SP ? 0 : u.page_begin * bpp;
   // Small pages: the segment's tokens tok0 .. tok_end - 1, its blocks counted from tok0.
   const int tok0 = u.page_begin * a.page_size;
-  const int tok_end =
-      static_cast<int>(min(static_cast<int64_t>(u.page_end) * a.page_size, static_cast<int64_t>(u.seq_len)));
+  // The schedule's last page may reach past the table's last token.
+  const int tok_end = static_cast<int>(
+      min(static_cast<int64_t>(u.page_end) * a.page_size, static_cast<int64_t>(SP ? min(u.seq_len, a.table_tokens) : 0)));
   const int blk_end = SP ? (tok_end - tok0 + kBlock - 1) / kBlock
                          : min(u.page_end * bpp, (u.seq_len + kBlock - 1) / kBlock);
   // This wave's blocks: blk_begin + wave + W * i, i < nblk.
@@ -1454,7 +1462,7 @@ __global__ void __launch_bounds__((uniform_waves<E, D, NT>() * 64), (mfma_waves_
   __shared__ __attribute__((
       aligned(16))) char lds[MfmaLds<D, NT, W, dma_staged<KVF, D, NT>(), kDmaStages, E::kBytes>::kBytes];
   __shared__ int s_last[1];
-  fetch_args<dma_staged<KVF, D, NT>()>(a);
+  fetch_args<kSmallPages<KVF>>(a);
   // q and the first block-table window depend on the unit alone: they are
   // issued before the kernel waits for seq_lens, so the first K/V loads
   // follow one memory round trip after it instead of two.
@@ -1502,7 +1510,7 @@ __global__ void __launch_bounds__(2 * kThreads, (mfma_waves_per_eu<D, NT>()))
   // Both halves hold the same sequence and split, so they agree on whether
   // there is work, whether it is final and how many segments the unit has:
   // they pass the same workgroup barriers.
-  fetch_args<dma_staged<KVF, D, NT>()>(a);
+  fetch_args<kSmallPages<KVF>>(a);
   // q and the first block-table window before seq_lens (decode_mfma_kernel).
   Unit u = decode_unit_paired_ids(a, half);
   QFrag<NT, qk_chunks<E, D>()> q;
@@ -1545,14 +1553,14 @@ __global__ void __launch_bounds__(2 * kThreads, (mfma_waves_per_eu<D, NT>()))
 
 __device__ __forceinline__ int seq_pages(const DecodeArgs& a, int b) {
   const int raw = a.seq_lens[b];
-  const int len = min(raw, a.max_len);
+  const int len = clamped_len(a, raw);
   return len > 0 ? (len + a.page_size - 1) / a.page_size : 0;
 }
 
 // seq_pages for a wave-uniform b: one scalar load.
 __device__ __forceinline__ int seq_pages_uniform(const DecodeArgs& a, int b) {
   const int raw = as_constant(a.seq_lens)[b];
-  const int len = min(raw, a.max_len);
+  const int len = clamped_len(a, raw);
   return len > 0 ? (len + a.page_size - 1) / a.page_size : 0;
 }
 
@@ -1635,10 +1643,6 @@ struct Start {
   // the batch when contexts are short).
   uint64_t empties[kScanChunks];
 };
-
-__device__ __forceinline__ int clamped_len(const DecodeArgs& a, int raw) {
-  return min(raw, a.max_len);
-}
 
 __device__ __forceinline__ int pages_of(const DecodeArgs& a, int len) {
   return len > 0 ? (len + a.page_size - 1) / a.page_size : 0;
@@ -1853,7 +1857,7 @@ __global__ void __launch_bounds__((PAIR * balanced_waves<KVF, D, NT, PAIR>() * 6
   using Lds = MfmaLds<D, NT, W, dma_staged<KVF, D, NT>()>;
   __shared__ __attribute__((aligned(16))) char lds[PAIR * Lds::kBytes];
   __shared__ int s_last[PAIR];
-  fetch_args<dma_staged<KVF, D, NT>()>(a);
+  fetch_args<kSmallPages<KVF>>(a);
   // A compile-time 0 with PAIR == 1, so the LDS base stays a constant.
   const int half = PAIR == 2 ? wave_id() / W : 0;
   const int hp = a.num_kv_heads * a.head_groups / PAIR;  // list units per sequence
@@ -2345,7 +2349,7 @@ __global__ void __launch_bounds__(64) decode_merge_kernel(const DecodeArgs a, in
   const int b = bh / a.num_q_heads;
   const int lane = __lane_id();
   const int raw = a.seq_lens[b];
-  const int seq_len = min(raw, a.max_len);
+  const int seq_len = clamped_len(a, raw);
   const int num_pages = seq_len > 0 ? (seq_len + a.page_size - 1) / a.page_size : 0;
   const int active = min(a.num_splits, (num_pages + a.pages_per_split - 1) / a.pages_per_split);
   S* out = static_cast<S*>(a.out) + static_cast<int64_t>(bh) * head_dim;
@@ -2426,7 +2430,7 @@ __global__ void __launch_bounds__(64) decode_merge_balanced_kernel(const DecodeA
 template <typename E, int D, int NT, int LDS>
 __device__ __forceinline__ void cascade_unit(const DecodeArgs& a, int idx, char (&lds)[LDS]) {
   static_assert(MfmaLds<D, NT, kWaves, dma_staged<E, D, NT>()>::kBytes <= LDS);
-  fetch_args<dma_staged<E, D, NT>()>(a);
+  fetch_args(a);
   Unit u = decode_unit_ids(a, idx);
   const int wave = wave_id();
   QFrag<NT, qk_chunks<E, D>()> q;
@@ -2529,17 +2533,13 @@ void set_division(int divisor, uint32_t* magic, int* shift) {
   *magic = static_cast<uint32_t>(((uint64_t{1} << *shift) + d - 1) / d);
 }
 
-// The longest sequence a table of max_pages columns holds.
-int table_tokens(int max_pages, int page_size) {
-  return static_cast<int>(std::min<int64_t>(static_cast<int64_t>(max_pages) * page_size, 0x7fffffff));
-}
-
-// The page sizes: the block table's, and the one the schedule counts in.
-void set_page_size(DecodeArgs& a, int table_page, int schedule_page) {
+// The block table's page size and width, and the page the schedule counts in.
+void set_page_size(DecodeArgs& a, int table_page, int table_pages, int schedule_page) {
   a.page_size = schedule_page;
   set_division(std::max(1, schedule_page / kBlock), &a.bpp_magic, &a.bpp_shift);
   a.table_page = table_page;
   set_division(table_page, &a.table_magic, &a.table_shift);
+  a.table_tokens = static_cast<int>(std::min<int64_t>(static_cast<int64_t>(table_pages) * table_page, 0x7fffffff));
 }
 
 // Shapes the MFMA kernels serve.
@@ -3265,9 +3265,8 @@ int decode_entry(kl_dtype dtype, bool kv8, void* out, const void* q, const void*
   a.num_q_heads = num_q_heads;
   a.num_kv_heads = num_kv_heads;
   a.group = num_q_heads / num_kv_heads;
-  set_page_size(a, page_size, p.page_size);
+  set_page_size(a, page_size, max_pages, p.page_size);
   a.max_pages = p.max_pages;
-  a.max_len = table_tokens(max_pages, page_size);
   a.num_splits = p.num_splits;
   a.pages_per_split = p.pages_per_split;
   a.head_groups = p.head_groups;
@@ -3472,7 +3471,6 @@ int cascade_launch(const DecodeArgs& base, const CascadePlan& cp, const int32_t*
   pre.group = batch * group;
   pre.num_q_heads = pre.num_kv_heads * pre.group;
   pre.max_pages = prefix_pages;
-  pre.max_len = table_tokens(prefix_pages, base.page_size);
   pre.num_splits = cp.pre.num_splits;
   pre.pages_per_split = cp.pre.pages_per_split;
   pre.head_groups = cp.pre.head_groups;
@@ -3484,7 +3482,6 @@ int cascade_launch(const DecodeArgs& base, const CascadePlan& cp, const int32_t*
   a.seq_lens = seq_lens;
   a.bt_stride = bt_stride;
   a.max_pages = max_pages;
-  a.max_len = table_tokens(max_pages, base.page_size);
   a.num_splits = cp.suf.num_splits;
   a.pages_per_split = cp.suf.pages_per_split;
   a.head_groups = cp.suf.head_groups;
@@ -3601,7 +3598,7 @@ extern "C" int kl_cascade_decode_attention(kl_dtype dtype, void* out, const void
   a.num_q_heads = num_q_heads;
   a.num_kv_heads = num_kv_heads;
   a.group = num_q_heads / num_kv_heads;
-  set_page_size(a, page_size, page_size);
+  set_page_size(a, page_size, max_pages, page_size);
   a.grid = 0;
   a.paired = 0;
   a.arrivals = nullptr;
