@@ -1826,21 +1826,22 @@ __device__ __forceinline__ Unit list_unit(const DecodeArgs& a, int hp, int ui, i
 }
 
 // Waves per KV head of a balanced workgroup: four, or eight for FP8 caches at
-// head_dim 128 where the registers allow them. An FP8 block is half the bytes, so
-// four waves with a block each on its way leave a CU short of loads. Measured,
-// four -> eight (us, 128 head dims, FP8): 32/1 B=64 up to 8,192 tokens 31.2 ->
-// 27.0, B=16 18.1 -> 17.0, 16/4 B=32 up to 4,096 22.5 -> 19.3, 32/8 B=16 up to
-// 2,048 17.8 -> 16.7. With one head tile it pays only while the launch has no
-// more workgroups than CUs (wide_fp8): 8/1 B=300 up to 2,000 38.4 -> 44.6, 40/5
-// B=100 24.6 -> 26.4. Paired (16 waves) it spilled and lost: 32/8 B=64 of 4,096
-// 86.1 -> 90.4. Small pages in 16 bits lost too: 32/8 B=32 page 8 29.6 -> 32.4.
-template <typename KVF, int D, int NT, int PAIR>
+// head_dim 128 while the launch has no more workgroups than CUs (wide_fp8). An
+// FP8 block is half the bytes, so four waves with a block each on its way leave a
+// CU short of loads; more workgroups fill it themselves, and eight waves of two
+// head tiles leave it room for one only. Measured, four -> eight (us, 128 head
+// dims, FP8): 32/1 B=64 up to 8,192 tokens 31.0 -> 26.7, B=100 41.4 -> 35.1, 16/4
+// B=32 up to 4,096 22.5 -> 19.3, 32/8 B=16 up to 2,048 19.3 -> 18.4; beyond: 32/1
+// B=260 of 4,096 94.7 -> 105.5, 8/1 B=300 up to 2,000 38.4 -> 44.6, 40/5 B=100
+// 24.6 -> 26.4. Paired (16 waves) it spilled and lost: 32/8 B=64 of 4,096 86.1 ->
+// 90.4. Small pages in 16 bits lost too: 32/8 B=32 page 8 29.6 -> 32.4.
+template <typename KVF>
 constexpr int balanced_waves() {
-  return kEightWaves<KVF> || (KVF::kBytes == 1 && D == 128 && NT == 2) ? 8 : kWaves;
+  return kEightWaves<KVF> ? 8 : kWaves;
 }
 template <typename KVF, int D, int NT, int PAIR>
 constexpr int balanced_waves_per_eu() {
-  const int waves = PAIR * balanced_waves<KVF, D, NT, PAIR>();
+  const int waves = PAIR * balanced_waves<KVF>();
   return std::max(mfma_waves_per_eu<D, NT>(), waves / 4);
 }
 
@@ -1850,10 +1851,10 @@ constexpr int balanced_waves_per_eu() {
 // of every token row, as in decode_mfma_paired_kernel). Half h of segment
 // (list workgroup w, list unit u) owns partial slot (w + u) * 2 + h.
 template <typename E, typename KVF, int D, int NT, int PAIR>
-__global__ void __launch_bounds__((PAIR * balanced_waves<KVF, D, NT, PAIR>() * 64),
+__global__ void __launch_bounds__((PAIR * balanced_waves<KVF>() * 64),
                                   (balanced_waves_per_eu<KVF, D, NT, PAIR>()))
     decode_mfma_balanced_kernel(const DecodeArgs a) {
-  constexpr int W = balanced_waves<KVF, D, NT, PAIR>();
+  constexpr int W = balanced_waves<KVF>();
   using Lds = MfmaLds<D, NT, W, dma_staged<KVF, D, NT>()>;
   __shared__ __attribute__((aligned(16))) char lds[PAIR * Lds::kBytes];
   __shared__ int s_last[PAIR];
@@ -3100,8 +3101,8 @@ int balanced_charge(int page_size, int head_dim, int kv_bytes, int paired, int h
       std::min<int64_t>(kMaxSegmentCharge, cdiv(kSegmentStartBytes + 2 * partial_bytes, page_bytes)));
 }
 
-// Whether an unpaired balanced launch of an FP8 cache with one head tile takes
-// eight waves per unit (balanced_waves).
+// Whether an unpaired balanced launch of an FP8 cache at head_dim 128 takes eight
+// waves per unit (balanced_waves).
 bool wide_fp8(const DecodeArgs& a) { return a.grid <= current_cu_count(); }
 
 template <typename E, typename KVF>
@@ -3122,21 +3123,19 @@ int launch_balanced(DecodeArgs a, int head_dim, hipStream_t stream) {
         // more than the 256 registers per lane of an 8-wave workgroup.
         if constexpr (D <= 128 && NT == 1 && !kSmallPages<KVF>) {
           decode_mfma_balanced_kernel<E, KVF, D, NT, 2>
-              <<<grid, 2 * balanced_waves<KVF, D, NT, 2>() * 64, 0, stream>>>(a);
+              <<<grid, 2 * kThreads, 0, stream>>>(a);
         } else {
           return fail(KL_ERR_UNSUPPORTED, "paired balanced decode needs head_dim <= 128 and <= 16 heads per workgroup");
         }
       } else {
-        if constexpr (KVF::kBytes == 1 && D == 128 && NT == 1) {
+        if constexpr (KVF::kBytes == 1 && D == 128) {
           if (wide_fp8(a)) {
             using W8 = EightWaves<KVF>;
-            decode_mfma_balanced_kernel<E, W8, D, NT, 1>
-                <<<grid, balanced_waves<W8, D, NT, 1>() * 64, 0, stream>>>(a);
+            decode_mfma_balanced_kernel<E, W8, D, NT, 1><<<grid, balanced_waves<W8>() * 64, 0, stream>>>(a);
             return KL_OK;
           }
         }
-        decode_mfma_balanced_kernel<E, KVF, D, NT, 1>
-            <<<grid, balanced_waves<KVF, D, NT, 1>() * 64, 0, stream>>>(a);
+        decode_mfma_balanced_kernel<E, KVF, D, NT, 1><<<grid, kThreads, 0, stream>>>(a);
       }
       return KL_OK;
     } else {
