@@ -1475,7 +1475,7 @@ __global__ void __launch_bounds__((uniform_waves<E, D, NT>() * 64), (mfma_waves_
   unit_pages(a, u);
   if (u.page_begin >= u.page_end) {
     wait_vmcnt<0>();  // the window loads write this workgroup's LDS
-    if (u.split == 0 && u.seq_len <= 0 && (a.num_splits == 1 || a.arrivals != nullptr)) {
+    if (u.split == 0 && u.seq_len <= 0 && (a.num_splits == 1 || a.arrivals != nullptr) && !a.force_partial) {
       write_zero_heads<typename E::S, E>(a, u, D, threadIdx.x, blockDim.x);
     }
     return;  // a split past the end of its sequence has no work
@@ -1524,7 +1524,7 @@ __global__ void __launch_bounds__(2 * kThreads, (mfma_waves_per_eu<D, NT>()))
     // The other half's segment passes two workgroup barriers: pass them too.
     __syncthreads();
     __syncthreads();
-    if (u.split == 0 && u.seq_len <= 0 && (a.num_splits == 1 || a.arrivals != nullptr)) {
+    if (u.split == 0 && u.seq_len <= 0 && (a.num_splits == 1 || a.arrivals != nullptr) && !a.force_partial) {
       write_zero_heads<typename E::S, E>(a, u, D, threadIdx.x - half * kThreads, kThreads);
     }
     return;
@@ -2413,8 +2413,8 @@ __global__ void __launch_bounds__(64) decode_merge_balanced_kernel(const DecodeA
 // the MFMA segment with all sequences' query heads of a KV head folded into
 // one group (q_fold), so each workgroup streams the prefix once for up to 32
 // query rows of many sequences; the suffix pass is the plain split decode.
-// Both run in one launch and write fp32 partials, and a merge kernel combines
-// them by the LSE rule.
+// Both write fp32 partials, and a merge kernel combines them by the LSE rule. They
+// run in one launch unless the own tokens are many and pair (kPairedOwnTokens).
 
 // Both passes in one launch: the first pre_wgs workgroups take the prefix's
 // units, the rest the sequences' own, each as decode_mfma_kernel would. The
@@ -2428,6 +2428,17 @@ __global__ void __launch_bounds__(64) decode_merge_balanced_kernel(const DecodeA
 // 64/8/128 bf16 B=16 16,384 + 1,024 47.9 -> 44.4, 32/8/128 B=4 2,000 + 300 18.5
 // -> 13.7. The own tokens first: 54.6; twice the prefix splits: 50.6; own
 // splits of 32 pages: 51.8. NTP, NTS: head tiles of the two passes.
+//
+// This launch has no KV-head pairs: with 8-wave workgroups a CU would hold one.
+// Where the own pass pairs (a full batch) and streams long sequences, pairs are
+// worth more than the overlap and each pass keeps a launch of its own. Measured, a
+// launch per pass -> one (us, 32/8/128 fp16, even own lengths): B=64 own 1,024
+// 55.7 -> 51.5, 2,048 94.8 -> 92.9, 4,096 172.6 -> 176.3, 8,192 328 -> 340, B=128
+// 4,096 332 -> 343; head_dim 64 B=128 4,096 + 4,096 205 -> 213. Uneven lengths sway
+// it either way (B=64 up to 4,096 115.5 -> 113.5, up to 8,192 227 -> 233, up to
+// 16,384 402 -> 380).
+constexpr int kPairedOwnTokens = 4096;  // tokens that the own block table holds
+
 template <typename E, int D, int NT, int LDS>
 __device__ __forceinline__ void cascade_unit(const DecodeArgs& a, int idx, char (&lds)[LDS]) {
   static_assert(MfmaLds<D, NT, kWaves, dma_staged<E, D, NT>()>::kBytes <= LDS);
@@ -2956,7 +2967,7 @@ int make_plan(const Options& opt, kl_dtype dtype, int batch, int num_q_heads, in
   // Two adjacent KV heads per 8-wave workgroup when the pairs alone give
   // every CU a workgroup (one 8-wave workgroup per CU is the register budget)
   // and the 4-wave kernel fits two waves per SIMD (head_dim <= 128).
-  p->paired = mfma16 && whole_blocks && !partials && opt.pairing() && num_kv_heads % 2 == 0 && head_dim <= 128 && units * s / 2 >= cus;
+  p->paired = mfma16 && whole_blocks && opt.pairing() && num_kv_heads % 2 == 0 && head_dim <= 128 && units * s / 2 >= cus;
   if (s > 1 || partials) {
     const size_t rows = static_cast<size_t>(batch) * num_q_heads * s;
     p->o_bytes = align_up(rows * head_dim * sizeof(float));
@@ -3491,8 +3502,21 @@ int cascade_launch(const DecodeArgs& base, const CascadePlan& cp, const int32_t*
       prefix_pages > 0 ? static_cast<int64_t>(pre.num_kv_heads) * pre.head_groups * pre.num_splits : 0;
   const int64_t wgs = pre_wgs + static_cast<int64_t>(batch) * a.num_kv_heads * a.head_groups * a.num_splits;
   if (wgs > 0x7fffffffLL) return fail(KL_ERR_UNSUPPORTED, "too many workgroups");
+  const bool pass_by_pass =
+      cp.suf.paired && static_cast<int64_t>(max_pages) * base.page_size >= kPairedOwnTokens;
+  if (pass_by_pass && pre_wgs > 0) {
+    pre.paired = cp.pre.paired ? 1 : 0;
+    int st = launch_uniform_mfma<E, E>(pre, head_dim, static_cast<unsigned>(pre_wgs), stream);
+    if (st != KL_OK) return st;
+    st = check_launch("cascade prefix pass launch");
+    if (st != KL_OK) return st;
+  }
   int st = dispatch_mfma(head_dim, a.heads_per_wg, [&](auto d, auto nts) -> int {
     constexpr int D = decltype(d)::value, NTS = decltype(nts)::value;
+    if (pass_by_pass) {
+      a.paired = 1;
+      return launch_uniform_mfma<E, E>(a, head_dim, static_cast<unsigned>(wgs - pre_wgs), stream);
+    }
     auto launch = [&](auto ntp) {
       cascade_decode_kernel<E, D, decltype(ntp)::value, NTS>
           <<<static_cast<unsigned>(wgs), kThreads, 0, stream>>>(pre, a, static_cast<int>(pre_wgs));

@@ -1,4 +1,4 @@
-"""Cascade decode's two passes in one launch: every pairing of their head tiles
+"""Cascade decode's two passes, in one launch or (long own tables of full batches) two: every pairing of their head tiles
 (one tile or two, i.e. up to 16 or more query heads per workgroup), the edges of
 blocks and splits on both sides, empty prefixes and empty own parts, and merges
 of more partials than one round loads."""
@@ -39,3 +39,17 @@ def test_many_partials(gpu_ops, head_dim):
 def test_no_prefix_pages(gpu_ops):
     q, c = random_cascade_problem(0, OWN, 32, 8, 128, 16, dtype=torch.float16, device="cuda")
     check(run(gpu_ops, q, c), expected(q, c), torch.float16)
+
+
+@pytest.mark.parametrize("head_dim", [32, 64, 128])
+@pytest.mark.parametrize("prefix", [0, 33, 300])
+@pytest.mark.parametrize(("hq", "hkv"), [(64, 64), (192, 64), (1536, 64)], ids=["one head", "tiles 2/1", "2/2"])
+def test_long_own_tables_of_full_batches(gpu_ops, head_dim, prefix, hq, hkv):
+    """8 x 64 units pair, and tables of 4,096 tokens take a launch per pass; 4,080
+    and less take one. The results of both match the oracle, empty rows too."""
+    for longest in (4096, 4080):
+        own = [longest, 0, 1, 16, 17, 65, 300, 129]
+        if hq > 192:
+            own[6] = 5
+        q, c = random_cascade_problem(prefix, own, hq, hkv, head_dim, 16, dtype=torch.float16, device="cuda", seed=prefix + hq)
+        check(run(gpu_ops, q, c), expected(q, c), torch.float16)
