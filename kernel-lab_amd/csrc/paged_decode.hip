@@ -2569,6 +2569,48 @@ bool small_pages_fit(int max_pages, int page_size) {
   return max_pages <= 0x7fffffff / 4 && static_cast<int64_t>(max_pages) * page_size <= 0x7fffffff - 2 * kBlock;
 }
 
+// Whether fp32 and small-page batches of short sequences run on the VALU kernel,
+// by the longest sequence their tables allow. An MFMA workgroup spends a segment's
+// start, its cross-wave merge and 16-row tiles on a unit of any size, and a CU holds
+// one or two; a VALU workgroup is small, and its work is tokens x query heads of
+// the unit, so it wins while that product is small and the units fill the device
+// several times over, or where one query head reads a few blocks. Of 1,788 points
+// measured (8 KV heads, batch 4 .. 500, tables of T = 24 .. 1,024 tokens, one to
+// eight heads per KV head, even lengths and lengths up to T) the choice was more
+// than 10 % slower than the VALU kernel at 11, the worst 28 %, and nowhere more than
+// 28 % off the fastest of the two kernels and schedules.
+// Measured (us, MFMA -> VALU):
+//   fp32 8/8/64 B=128 T=512 42.5 -> 36.6; 8/8/128 B=128 T=64 25.4 -> 12.8, T=256 48.0
+//     -> 35.4; 32/8/128 B=128 T=64 26.2 -> 23.5; 8/8/256 B=128 T=128 65.1 -> 36.6; the
+//     other way 8/8/128 B=64 T=256 23 -> 33, 64/8/128 B=128 T=64 27 -> 43;
+//   page 8, bf16 8/8/64 B=128 T=512 38.3 -> 34.0, B=64 T=128 13.6 -> 9.1, B=8 T=64
+//     7.6 -> 5.7; 8/8/128 B=128 T=128 18.4 -> 15.7; 8/8/256 B=128 T=256 53.8 -> 39.0;
+//     the other way 8/8/128 B=64 T=256 15.7 -> 19.3, 32/8/64 B=64 T=64 12.6 -> 15.9.
+// units: (sequence, KV head) pairs, each with its given splits.
+bool valu_path(kl_dtype dtype, int head_dim, int group, int64_t units, int64_t tokens, int cus) {
+  const bool fp32 = dtype == KL_DTYPE_F32;
+  if (group == 1 && tokens <= (fp32 ? 48 : head_dim <= 64 ? 128 : head_dim == 128 ? 64 : 48)) return true;
+  struct Line {
+    int max_group, num, den, most;  // tokens x heads <= min(most, units * num / den)
+  };
+  const Line line = fp32 ? (head_dim <= 64    ? Line{4, 2, 3, 1024}
+                            : head_dim == 128 ? Line{4, 1, 3, 512}
+                                              : Line{8, 1, 3, 512})
+                         : (head_dim <= 64    ? Line{2, 3, 2, 2048}
+                            : head_dim == 128 ? Line{2, 1, 4, 512}
+                                              : Line{4, 1, 3, 512});
+  const int rounds = group > 2 || (!fp32 && head_dim == 128) ? 3 : 2;
+  return group <= line.max_group && units >= static_cast<int64_t>(rounds) * cus &&
+         tokens * group <= std::min<int64_t>(line.most, units * line.num / line.den);
+}
+
+// Longest table, in tokens, that small pages serve with uniform splits: the
+// balanced schedule's ranges of at least 8 pages of 16 tokens walk several short
+// units one after the other, where uniform splits give each a workgroup. Measured
+// (us, bf16 page 8, balanced -> uniform): 32/8/128 B=8 of 16 .. 32 tokens 19.1 -> 6.1,
+// B=32 of 256 .. 512 21.3 -> 14.7, B=128 of 512 .. 1,024 92.0 -> 76.0.
+constexpr int kUniformSmallPageTokens = 1024;
+
 // Switches for A/B measurements and tests; unset, the library behaves as
 // planned below. They are read from the environment once per process, at
 // the first call that needs them, and again by
@@ -2824,11 +2866,20 @@ int make_plan(const Options& opt, kl_dtype dtype, int batch, int num_q_heads, in
   // counted in pages of one block when the planner chooses it, so the rules
   // below see the lengths they were measured at, and in the table's own pages
   // when the caller gives the split count, as the original counts them. Tables
-  // beyond small_pages_fit keep the VALU kernel.
-  const bool mfma = use_mfma && mfma_path(dtype, head_dim) && (whole_blocks || small_pages_fit(max_pages, page_size));
+  // beyond small_pages_fit keep the VALU kernel, and so do short sequences of
+  // small pages and of fp32 (valu_path).
+  const int group = num_q_heads / num_kv_heads;
+  const int cus = cu_count > 0 ? cu_count : 256;
+  const int64_t table_tokens = static_cast<int64_t>(max_pages) * page_size;
+  const int given = std::max(1, num_splits);
+  const bool short_valu =
+      (dtype == KL_DTYPE_F32 || !whole_blocks) &&
+      valu_path(dtype, head_dim, group, static_cast<int64_t>(batch) * num_kv_heads * given, cdiv(table_tokens, given), cus);
+  const bool mfma = use_mfma && mfma_path(dtype, head_dim) && !short_valu &&
+                    (whole_blocks || small_pages_fit(max_pages, page_size));
   p->mfma = mfma;
   if (mfma && !whole_blocks && num_splits <= 0) {
-    max_pages = static_cast<int>(cdiv(static_cast<int64_t>(max_pages) * page_size, kBlock));
+    max_pages = static_cast<int>(cdiv(table_tokens, kBlock));
     page_size = kBlock;
   }
   p->page_size = page_size;
@@ -2837,12 +2888,10 @@ int make_plan(const Options& opt, kl_dtype dtype, int batch, int num_q_heads, in
   if (!mfma && !valu_head_dim_ok(dtype, head_dim)) {
     return fail(KL_ERR_UNSUPPORTED, "head_dim must be 16, 32, 64, 128 or 256");
   }
-  const int group = num_q_heads / num_kv_heads;
   head_tiling(mfma, head_dim, group, &p->heads_per_wg, &p->head_groups);
   const int pages = std::max(max_pages, 1);
   p->grid = 0;
   p->paired = false;
-  const int cus = cu_count > 0 ? cu_count : 256;
   const int64_t units = std::max<int64_t>(1, static_cast<int64_t>(batch) * num_kv_heads * p->head_groups);
   if (num_splits == KL_SPLITS_BALANCED && (!mfma16 || partials)) num_splits = 0;  // uniform splits only
   // The balanced schedule runs in KV-head pairs (8-wave workgroups) on
@@ -2885,8 +2934,9 @@ int make_plan(const Options& opt, kl_dtype dtype, int batch, int num_q_heads, in
   // ctx 512 11.24 -> 9.92, ctx 4096 16.28 -> 13.20, ctx 32768 33.04 -> 31.76;
   // 8/1/128 ctx 32768 26.08 -> 16.40.
   const bool single = batch == 1 && !long_pairs;
+  const bool short_units = !whole_blocks && table_tokens <= kUniformSmallPageTokens;
   const bool automatic =
-      num_splits == 0 && !single && list_fits &&
+      num_splits == 0 && !single && !short_units && list_fits &&
       (units < cus || (full_batch_choice < 0 ? full_default : full_batch_choice == 1));
   const bool balance = requested || automatic;
   const bool pair_balanced = pairable && balance;

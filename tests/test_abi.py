@@ -267,6 +267,16 @@ def test_small_page_tables_stay_within_the_index_arithmetic(dtype, page, max_pag
     assert splits == (32 if mfma else 16)
 
 
+@pytest.mark.parametrize(
+    ("batch", "tokens", "splits"),
+    [(8, 1024, 4), (8, 1032, 0), (32, 1024, 1), (32, 1032, 0)],
+)
+def test_short_small_page_tables_take_uniform_splits(batch, tokens, splits):
+    """Pages of 8 tokens: tables of up to 1,024 tokens take uniform splits (of at
+    least 16 blocks of 16 tokens), longer ones the balanced schedule (0)."""
+    assert ops.plan_decode(torch.float16, batch, 32, 8, 128, 8, tokens // 8, 0, 256)[0] == splits
+
+
 def test_planner_rejects_bad_shapes():
     with pytest.raises(ValueError, match="multiple"):
         ops.plan_decode(torch.float16, 2, 3, 2, 128, 16, 4)
