@@ -2554,6 +2554,9 @@ void set_page_size(DecodeArgs& a, int table_page, int table_pages, int schedule_
   a.table_tokens = static_cast<int>(std::min<int64_t>(static_cast<int64_t>(table_pages) * table_page, 0x7fffffff));
 }
 
+// Most query heads of a GQA group that one MFMA workgroup takes.
+int mfma_heads_cap(int group, int head_dim) { return (group > 16 && head_dim <= 128) ? 32 : 16; }
+
 // Shapes the MFMA kernels serve.
 bool mfma_path(kl_dtype dtype, int head_dim) {
   if (head_dim == 64 || head_dim == 128 || head_dim == 256) return true;
@@ -2567,6 +2570,14 @@ bool mfma_path(kl_dtype dtype, int head_dim) {
 // index is rounded up by as much as two blocks before it is clamped.
 bool small_pages_fit(int max_pages, int page_size) {
   return max_pages <= 0x7fffffff / 4 && static_cast<int64_t>(max_pages) * page_size <= 0x7fffffff - 2 * kBlock;
+}
+
+// Whether `splits` partials per head lie within the MFMA kernels' reach: a
+// workgroup stores its heads' rows, `splits` rows of fp32 apart, at 32-bit byte
+// offsets through a buffer resource of 2^31 - 1 bytes, which drops what is beyond.
+bool partials_fit(int head_dim, int group, int splits) {
+  const int heads = std::min(group, mfma_heads_cap(group, head_dim));
+  return (static_cast<int64_t>(heads - 1) * splits + 1) * head_dim * 4 <= 0x7fffffff;
 }
 
 // Whether fp32 and small-page batches of short sequences run on the VALU kernel,
@@ -2814,7 +2825,7 @@ bool valu_head_dim_ok(kl_dtype dtype, int head_dim) {
 void head_tiling(bool mfma, int head_dim, int group, int* per_wg, int* groups) {
   int cap;
   if (mfma) {
-    cap = (group > 16 && head_dim <= 128) ? 32 : 16;
+    cap = mfma_heads_cap(group, head_dim);
   } else {
     cap = 8;
   }
@@ -2867,7 +2878,7 @@ int make_plan(const Options& opt, kl_dtype dtype, int batch, int num_q_heads, in
   // below see the lengths they were measured at, and in the table's own pages
   // when the caller gives the split count, as the original counts them. Tables
   // beyond small_pages_fit keep the VALU kernel, and so do short sequences of
-  // small pages and of fp32 (valu_path).
+  // small pages and of fp32 (valu_path) and split counts beyond partials_fit.
   const int group = num_q_heads / num_kv_heads;
   const int cus = cu_count > 0 ? cu_count : 256;
   const int64_t table_tokens = static_cast<int64_t>(max_pages) * page_size;
@@ -2876,6 +2887,7 @@ int make_plan(const Options& opt, kl_dtype dtype, int batch, int num_q_heads, in
       (dtype == KL_DTYPE_F32 || !whole_blocks) &&
       valu_path(dtype, head_dim, group, static_cast<int64_t>(batch) * num_kv_heads * given, cdiv(table_tokens, given), cus);
   const bool mfma = use_mfma && mfma_path(dtype, head_dim) && !short_valu &&
+                    partials_fit(head_dim, group, std::min(given, std::max(max_pages, 1))) &&
                     (whole_blocks || small_pages_fit(max_pages, page_size));
   p->mfma = mfma;
   if (mfma && !whole_blocks && num_splits <= 0) {
