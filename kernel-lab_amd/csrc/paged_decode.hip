@@ -2580,6 +2580,10 @@ bool partials_fit(int head_dim, int group, int splits) {
   return (static_cast<int64_t>(heads - 1) * splits + 1) * head_dim * 4 <= 0x7fffffff;
 }
 
+// Threads of a grid; a launch of 2^32 and more wraps without an error (a grid of
+// 8.8 million workgroups of 512 threads ran 2^32 threads short).
+bool grid_fits(int64_t workgroups, int threads) { return workgroups * threads <= 0xffffffffLL; }
+
 // Whether fp32 and small-page batches of short sequences run on the VALU kernel,
 // by the longest sequence their tables allow. An MFMA workgroup spends a segment's
 // start, its cross-wave merge and 16-row tiles on a unit of any size, and a CU holds
@@ -2878,7 +2882,8 @@ int make_plan(const Options& opt, kl_dtype dtype, int batch, int num_q_heads, in
   // below see the lengths they were measured at, and in the table's own pages
   // when the caller gives the split count, as the original counts them. Tables
   // beyond small_pages_fit keep the VALU kernel, and so do short sequences of
-  // small pages and of fp32 (valu_path) and split counts beyond partials_fit.
+  // small pages and of fp32 (valu_path), split counts beyond partials_fit, and
+  // fp32 grids too large for eight waves a workgroup (uniform_waves).
   const int group = num_q_heads / num_kv_heads;
   const int cus = cu_count > 0 ? cu_count : 256;
   const int64_t table_tokens = static_cast<int64_t>(max_pages) * page_size;
@@ -2886,8 +2891,13 @@ int make_plan(const Options& opt, kl_dtype dtype, int batch, int num_q_heads, in
   const bool short_valu =
       (dtype == KL_DTYPE_F32 || !whole_blocks) &&
       valu_path(dtype, head_dim, group, static_cast<int64_t>(batch) * num_kv_heads * given, cdiv(table_tokens, given), cus);
+  const int64_t mfma_units =
+      static_cast<int64_t>(batch) * num_kv_heads * cdiv(group, mfma_heads_cap(group, head_dim));
+  const bool fp32_grid_fits =
+      head_dim > 128 || group > 16 || grid_fits(mfma_units * std::min(given, std::max(max_pages, 1)), 2 * kThreads);
   const bool mfma = use_mfma && mfma_path(dtype, head_dim) && !short_valu &&
                     partials_fit(head_dim, group, std::min(given, std::max(max_pages, 1))) &&
+                    (dtype != KL_DTYPE_F32 || fp32_grid_fits) &&
                     (whole_blocks || small_pages_fit(max_pages, page_size));
   p->mfma = mfma;
   if (mfma && !whole_blocks && num_splits <= 0) {
@@ -3235,7 +3245,7 @@ int launch_typed(DecodeArgs& a, int head_dim, bool mfma, hipStream_t stream) {
     if constexpr (!std::is_same_v<E, F32>) return launch_balanced<E, KVF>(a, head_dim, stream);
   }
   const int64_t wgs = static_cast<int64_t>(a.batch) * a.num_kv_heads * a.head_groups * a.num_splits;
-  if (wgs > 0x7fffffffLL) return fail(KL_ERR_UNSUPPORTED, "too many workgroups");
+  if (wgs > 0x7fffffffLL || !grid_fits(wgs, kThreads)) return fail(KL_ERR_UNSUPPORTED, "too many workgroups");
   if (mfma && a.num_splits > 1) {
     a.arrivals = fused_merge_counters(a, static_cast<int64_t>(a.batch) * a.num_kv_heads * a.head_groups, stream);
   }

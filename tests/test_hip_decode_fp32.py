@@ -45,3 +45,20 @@ def test_fp32_mfma_is_no_further_from_64_bits_than_torch(gpu_ops, head_dim):
         w = torch.softmax(q[b].cpu().double().reshape(2, 4, head_dim) @ k.transpose(1, 2) * head_dim**-0.5, -1)
         want = (w @ v).reshape(8, head_dim)
         assert (out[b] - want).norm() <= 4e-7 * want.norm()
+
+
+def test_more_workgroups_than_eight_waves_allow(gpu_ops):
+    """1,100,000 sequences of 8 KV heads, all but seven empty: a grid of 8.8 million
+    workgroups, which 512 threads each would take past 2^32. Tables of 1,040 tokens,
+    so the batch does not count as short."""
+    batch, lens_at = 1_100_000, [0, 1, 500_000, 1_048_575, 1_048_576, 1_048_577, 1_099_999]
+    g = torch.Generator(device="cuda").manual_seed(0)
+    q = torch.randn(batch, 8, 64, generator=g, device="cuda")
+    k, v = torch.randn(2, 1, 16, 8, 64, generator=g, device="cuda")
+    table = torch.zeros(batch, 65, dtype=torch.int32, device="cuda")
+    lens = torch.zeros(batch, dtype=torch.int32, device="cuda")
+    lens[lens_at] = 5
+    out = gpu_ops.paged_decode_attention(q, k, v, table, lens)
+    assert int((out != 0).any(-1).any(-1).sum()) == len(lens_at)
+    want = ref.paged_decode_attention(q[lens_at].cpu(), k.cpu(), v.cpu(), table[lens_at].cpu(), lens[lens_at].cpu())
+    decode_parity(out[lens_at], want, torch.float32)
