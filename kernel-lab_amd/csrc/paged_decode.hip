@@ -3574,8 +3574,12 @@ int cascade_launch(const DecodeArgs& base, const CascadePlan& cp, const int32_t*
       prefix_pages > 0 ? static_cast<int64_t>(pre.num_kv_heads) * pre.head_groups * pre.num_splits : 0;
   const int64_t wgs = pre_wgs + static_cast<int64_t>(batch) * a.num_kv_heads * a.head_groups * a.num_splits;
   if (wgs > 0x7fffffffLL) return fail(KL_ERR_UNSUPPORTED, "too many workgroups");
+  // A launch per pass: see kPairedOwnTokens, and where the two grids are too large for one.
   const bool pass_by_pass =
-      cp.suf.paired && static_cast<int64_t>(max_pages) * base.page_size >= kPairedOwnTokens;
+      (cp.suf.paired && static_cast<int64_t>(max_pages) * base.page_size >= kPairedOwnTokens) || !grid_fits(wgs, kThreads);
+  if (!grid_fits(pre_wgs, kThreads) || !grid_fits(wgs - pre_wgs, kThreads)) {
+    return fail(KL_ERR_UNSUPPORTED, "too many workgroups");
+  }
   if (pass_by_pass && pre_wgs > 0) {
     pre.paired = cp.pre.paired ? 1 : 0;
     int st = launch_uniform_mfma<E, E>(pre, head_dim, static_cast<unsigned>(pre_wgs), stream);
@@ -3586,7 +3590,7 @@ int cascade_launch(const DecodeArgs& base, const CascadePlan& cp, const int32_t*
   int st = dispatch_mfma(head_dim, a.heads_per_wg, [&](auto d, auto nts) -> int {
     constexpr int D = decltype(d)::value, NTS = decltype(nts)::value;
     if (pass_by_pass) {
-      a.paired = 1;
+      a.paired = cp.suf.paired ? 1 : 0;
       return launch_uniform_mfma<E, E>(a, head_dim, static_cast<unsigned>(wgs - pre_wgs), stream);
     }
     auto launch = [&](auto ntp) {

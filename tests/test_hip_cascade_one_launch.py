@@ -9,6 +9,7 @@ import pytest
 import torch
 
 from kernel_lab.kv_cache import random_cascade_problem
+from oracle import reference as ref
 from tests.test_hip_cascade import check, expected, run
 
 pytestmark = pytest.mark.gpu
@@ -53,3 +54,20 @@ def test_long_own_tables_of_full_batches(gpu_ops, head_dim, prefix, hq, hkv):
             own[6] = 5
         q, c = random_cascade_problem(prefix, own, hq, hkv, head_dim, 16, dtype=torch.float16, device="cuda", seed=prefix + hq)
         check(run(gpu_ops, q, c), expected(q, c), torch.float16)
+
+
+def test_grids_too_large_for_one_launch(gpu_ops):
+    """2,050,000 sequences of 8 heads: 16.4 million workgroups for the own tokens and
+    0.5 million for the prefix, together past 2^32 threads. Each takes a launch."""
+    batch, at = 2_050_000, [0, 1_000_000, 2_033_599, 2_033_600, 2_049_999]
+    g = torch.Generator(device="cuda").manual_seed(0)
+    q = torch.randn(batch, 8, 32, generator=g, device="cuda").half()
+    k, v = torch.randn(2, 2, 16, 8, 32, generator=g, device="cuda").half()
+    table = torch.ones(batch, 1, dtype=torch.int32, device="cuda")
+    lens = torch.full((batch,), 3, dtype=torch.int32, device="cuda")
+    prefix = torch.zeros(1, dtype=torch.int32, device="cuda"), torch.tensor([11], dtype=torch.int32, device="cuda")
+    out = gpu_ops.cascade_decode_attention(q, k, v, *prefix, table, lens)
+    assert (out != 0).any(-1).all()
+    want = ref.cascade_decode_attention(q[at].cpu().float(), k.cpu(), v.cpu(), prefix[0].cpu(), prefix[1].cpu(), table[at].cpu(),
+                                        lens[at].cpu())
+    check(out[at], want, torch.float16)
