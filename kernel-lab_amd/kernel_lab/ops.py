@@ -52,11 +52,13 @@ def _rows_view(x: torch.Tensor) -> torch.Tensor:
 
 def _carries_nothing(t: torch.Tensor) -> bool:
     """Whether a clone of t would hold no more than its values: no autograd
-    history, forward-mode tangent or subclass."""
+    history, forward-mode tangent or subclass. torch has no public question for
+    an open forward-mode level; where its private one is gone, none counts as
+    closed."""
     return (
         type(t) in (torch.Tensor, torch.nn.Parameter)
         and not (t.requires_grad and torch.is_grad_enabled())
-        and forward_ad._current_level < 0
+        and getattr(forward_ad, "_current_level", 0) < 0
     )
 
 

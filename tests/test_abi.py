@@ -340,3 +340,12 @@ def test_remembered_plan_follows_its_arguments():
     for _ in range(3):
         assert (ops.plan_decode(*a), ops.plan_decode(*b)) == first
     assert first[0] != first[1]
+
+
+def test_functional_norm_does_not_need_torchs_private_level(monkeypatch):
+    """The clone-free form asks torch for an open forward-mode level by a private
+    name; without that name every residual is cloned and nothing raises."""
+    residual = torch.ones(2, 4)
+    assert ops._carries_nothing(residual)
+    monkeypatch.delattr(torch.autograd.forward_ad, "_current_level")
+    assert not ops._carries_nothing(residual)
