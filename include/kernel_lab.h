@@ -126,9 +126,10 @@ int kl_rms_norm_grouped(kl_dtype dtype, void* out, const void* x, const void* re
  *                    detected on the device; full batches of more than 8
  *                    query heads per KV head take it only when the table
  *                    spans >= 256 pages; a single sequence takes uniform
- *                    splits of >= 8 pages); when page_size is
+ *                    splits of >= 8 pages; when page_size is
  *                    not a multiple of 16 the planner counts pages of
- *                    16 tokens, a count the caller gives its own pages
+ *                    16 tokens, a count the caller gives its own pages,
+ *                    and tables of up to 1,024 tokens take uniform splits)
  *   out_workspace    (host pointer) bytes of device workspace the launch needs
  *                    (0 when the launch needs none)
  */
@@ -161,8 +162,8 @@ int kl_paged_decode_plan(kl_dtype dtype, int batch, int num_q_heads, int num_kv_
  * NULL when that is 0. batch == 0 is a successful no-op.
  *
  * Split sequences are merged inside the decode kernel where the path allows
- * it (fp16/bf16, at most 8 query heads per KV head and head group, and a
- * sequence cut into few enough segments that one workgroup's merge stays
+ * it (the MFMA kernels of every dtype and cache, at most 8 query heads per KV
+ * head and head group, and a sequence cut into few enough segments that one workgroup's merge stays
  * short; otherwise a separate merge launch runs). The library keeps
  * per-device arrival counters (8 MiB) in regions that calls able to overlap
  * never share: an eager call uses its stream's region (64 streams per

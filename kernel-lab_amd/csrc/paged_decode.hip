@@ -15,9 +15,9 @@
 //                    a long sequence among short ones is spread over many
 //                    workgroups (chosen when units do not fill the device, or
 //                    on request).
-// A segment runs on four waves; its 16-token blocks go round-robin to the
-// waves, each wave keeps its own running max / normaliser / output, and the
-// waves merge through LDS at the end. Uniform splits on a device they fill
+// A segment runs on four waves (eight where uniform_waves and balanced_waves say
+// so); its 16-token blocks go round-robin to the waves, each wave keeps its own
+// running max / normaliser / output, and the waves merge through LDS at the end. Uniform splits on a device they fill
 // twice over run two segments per 8-wave workgroup, KV heads 2j and 2j+1 of
 // one sequence side by side (adjacent bytes of every token row). A segment that covers its whole unit
 // writes the final output; otherwise it writes an fp32 partial output and its
@@ -35,7 +35,8 @@
 //                   layout (lane = head, 4 consecutive tokens) is the B operand
 //                   layout, so P never leaves registers; P goes in as a 16-bit
 //                   high part and low part (k = the block's tokens twice), so
-//                   the weights keep ~17-21 bits. V is loaded the same
+//                   the weights keep ~17-21 bits (small pages: 24, see
+//                   fp32_weights). V is loaded the same
 //                   row-coalesced way, staged in LDS and read back transposed
 //                   (ds_read_b64_tr_b16) as the A operand.
 // Every K/V element is read from HBM once per unit and used by the whole GQA
@@ -53,11 +54,12 @@
 //                   tile's registers: neither touches LDS.
 // What bounds it: HBM on full batches, the longest sequence's workgroup on
 // ragged ones (uniform splits). Measured (us, VALU kernel -> this): 32/8/128
-// B=16 up to 4,096 tokens 384 -> 64, B=64 of 512 tokens 120 -> 47.6 (5.6 TB/s),
+// B=16 up to 4,096 tokens 403 -> 56.7, B=64 of 512 tokens 120 -> 47.6 (5.6 TB/s),
 // 32/1/128 B=16 up to 8,192 599 -> 43.6, 16/4/256 B=8 up to 4,096 200 -> 41.4,
 // 8/1/64 B=4 up to 512 62.7 -> 9.9.
 //
-// VALU path (shapes the MFMA paths do not take): lanes own 16-byte
+// VALU path (shapes the MFMA paths do not take, and short fp32 and small-page
+// sequences: valu_path): lanes own 16-byte
 // slices of a token's head dims; dot products reduce across the lanes of a
 // token; each lane keeps an online softmax per query head and lanes merge by
 // the log-sum-exp rule at the end.
@@ -197,7 +199,7 @@ __device__ __forceinline__ int table_column(const DecodeArgs& a, int tok) {
 // whole and coalesced, so HBM and the segment starts bound it as they do the
 // other caches; the addresses cost about 40 VALU instructions a block. Measured
 // (us, VALU kernel -> this): 32/8/128 bf16 page 8 B=32 up to 2,048 tokens 207 ->
-// 30.5.
+// 31.3.
 template <typename F>
 struct SmallPages : F {};
 template <typename KVF>
@@ -313,21 +315,6 @@ struct Mfma<BF16> {
   static __device__ __forceinline__ f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b),
                                                    c, 0, 0, 0);
-  }
-};
-
-// fp32 products, four 16x16x4 MFMAs: element j of the operands is k step j, in
-// which lane l supplies A[row l % 16][k = l / 16] and B[k = l / 16][col l % 16].
-// Which four values of the contraction a step takes is free as long as A and B
-// agree, so both operands keep the 16-bit ones' shape (a lane holds 16
-// consecutive bytes of its row).
-template <>
-struct Mfma<F32> {
-  static __device__ __forceinline__ f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
-    const f32x4 av = __builtin_bit_cast(f32x4, a), bv = __builtin_bit_cast(f32x4, b);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j], bv[j], c, 0, 0, 0);
-    return c;
   }
 };
 
@@ -785,7 +772,9 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
   // A padding slot of the last round (live false) loads through resources of
   // no records: the hardware answers with zeros and touches no memory, so no
   // load is still travelling when the waves meet at the merge's barrier
-  // (which waits for every outstanding load).
+  // (which waits for every outstanding load). Small pages have no such resource:
+  // their padding slots read the wave's last block again (one block of fp32, up
+  // to NS - 1 of 16 bits).
   //
   // table_load, block_src, first_src and load_half stand for either addressing:
   // a block's table entry (or the lane's entries), its source from that entry,
@@ -856,10 +845,15 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
     for (int t = 0; t < NT; ++t) {
       f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
       if constexpr (FP32) {
-        // Sums of four products (one MFMA), then a tree over them. One running
-        // sum over all of head_dim rounds more: 16 sequences of up to 4,096
-        // tokens at head_dim 128 were 4.7e-7 off 64 bits with it, 2.3e-7 with
-        // the tree, 3.4e-7 on the VALU kernel.
+        // v_mfma_f32_16x16x4_f32: lane l supplies A[row l % 16][k = l / 16] and
+        // B[k = l / 16][col l % 16]. Which four values of the contraction a step
+        // takes is free as long as A and B agree, so both operands keep the
+        // 16-bit ones' shape (a lane holds 16 consecutive bytes of its row) and
+        // element j is step j.
+        //
+        // Sums of four products (one MFMA), then a tree over them, as one running
+        // sum over all of head_dim rounds more. 16 sequences of up to 4,096 tokens
+        // at head_dim 128 are 1.7e-7 off 64 bits, 2.4e-7 on the VALU kernel (2-norm).
         f32x4 part[KC];
 #pragma unroll
         for (int c = 0; c < KC; ++c) {
@@ -1308,7 +1302,7 @@ constexpr int kArrivalCounters = 8192;   // units per region (8 MiB per device i
 // than the merge kernel (52.4 vs 49.8 us), and the merge code alone slowed
 // the two-tile kernel's main loop (46 -> 50 us), so those keep the merge kernel.
 constexpr int kFusedMergeMaxHeads = 8;
-// The last arriver's four waves merge the unit serially: each takes
+// The last arriver's waves (four or eight) merge the unit serially: each takes
 // cdiv(heads, 4) heads of `segments` partials, where the merge kernel gives
 // every (sequence, head) its own wave. Measured on MI355X (events, us, same
 // uniform splits, fused vs merge kernel), by heads per wave x segments: 8-16
@@ -2806,6 +2800,8 @@ uint32_t* fused_merge_counters(const DecodeArgs& a, int64_t units, hipStream_t s
   // workgroups per list unit on even lengths.
   const int64_t list_units = std::max<int64_t>(1, a.grid > 0 && a.paired ? units / 2 : units);
   const int64_t segments = a.grid > 0 ? cdiv(a.grid, list_units) : a.num_splits;
+  // Heads per wave at four waves, where the bound was measured; eight waves merge
+  // in no more than that.
   if (cdiv(a.heads_per_wg, kWaves) * segments > kFusedMergeMaxWork) return nullptr;
   return arrival_region(stream);
 }

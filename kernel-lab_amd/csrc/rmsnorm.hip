@@ -150,12 +150,9 @@ __device__ __forceinline__ void norm_row(typename E::S* out, const typename E::S
     a[k] = load_at<ALIGNED, P>(x, off[k]);
     if constexpr (HAS_RES) b[k] = load_at<ALIGNED, P>(res, off[k]);
   }
-  // As in rms_norm_reg_kernel: ahead of the reduction unless the registers are short.
-  constexpr bool kEarlyWeights = NPACK <= 4;
-  if constexpr (kEarlyWeights) {
+  // At most four packs: the weights travel through the reduction.
 #pragma unroll
-    for (int k = 0; k < NPACK; ++k) w[k] = load_at<ALIGNED, P>(weight, off[k]);
-  }
+  for (int k = 0; k < NPACK; ++k) w[k] = load_at<ALIGNED, P>(weight, off[k]);
   float sum_sq = 0.0f;
 #pragma unroll
   for (int k = 0; k < NPACK; ++k) {
@@ -183,7 +180,6 @@ __device__ __forceinline__ void norm_row(typename E::S* out, const typename E::S
   }
 #pragma unroll
   for (int k = 0; k < NPACK; ++k) {
-    if constexpr (!kEarlyWeights) w[k] = load_at<ALIGNED, P>(weight, off[k]);
     P o;
 #pragma unroll
     for (int j = 0; j < VEC; ++j) o.v[j] = E::from_f32((E::to_f32(a[k].v[j]) * rstd) * E::to_f32(w[k].v[j]));
@@ -321,8 +317,8 @@ __global__ void __launch_bounds__(kMaxThreads)
 }
 
 // Rows wider than the register-resident kernel holds (more than 8 packs per
-// thread at 1024 threads: 65,536 16-bit or 32,768 fp32 elements aligned, 8,192
-// unaligned). Two passes over the row with the rounded sum kept in LDS:
+// thread at 1024 threads, 4 unaligned: 65,536 16-bit or 32,768 fp32 elements
+// aligned, half of them unaligned). Two passes over the row with the rounded sum kept in LDS:
 //   pass 1  reads x (and the residual), forms the rounded sum, accumulates its
 //           squares, and keeps the sum of the row's first kStagedPacks packs in
 //           LDS (writing their residual now);
@@ -406,7 +402,7 @@ __global__ void __launch_bounds__(kMaxThreads)
 // 16.6 -> 4.6, 16,384 rows of 512 7.2 -> 6.8; 16 rows of 128 equal.
 constexpr int kRowsThreads = 256;
 
-template <typename E, int LANES, int NPACK, bool HAS_RES, bool ALIGNED>
+template <typename E, int LANES, bool HAS_RES, bool ALIGNED>
 __global__ void __launch_bounds__(kRowsThreads)
     rms_norm_rows_kernel(typename E::S* __restrict__ out, const typename E::S* __restrict__ x,
                          typename E::S* __restrict__ res, int64_t res_out, const typename E::S* __restrict__ weight,
@@ -414,7 +410,7 @@ __global__ void __launch_bounds__(kRowsThreads)
   const int64_t r = static_cast<int64_t>(blockIdx.x) * (kRowsThreads / LANES) + threadIdx.x / LANES;
   const bool live = r < rows;
   const int64_t row = live ? r : rows - 1;
-  norm_row<E, 16 / E::kBytes, NPACK, HAS_RES, ALIGNED>(
+  norm_row<E, 16 / E::kBytes, 1, HAS_RES, ALIGNED>(
       out + row * hidden, x + x_rows.x_of_row(row), HAS_RES ? res + row * hidden : nullptr,
       res_out, weight, hidden, eps, threadIdx.x % LANES, LANES, live, [](float v) { return lanes_sum<LANES>(v); });
 }
@@ -439,14 +435,13 @@ __global__ void __launch_bounds__(kMaxThreads)
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// Calls f(IntC<N>) with the smallest N of 1, 2, 4, 8 that holds npack.
+// Calls f(IntC<N>) with the smallest N of 2, 4, 8 that holds npack (a row of one
+// pack per thread is narrow enough for rms_norm_rows_kernel).
 template <int N>
 using IntC = std::integral_constant<int, N>;
 template <typename F>
 void with_packs(int npack, F&& f) {
-  if (npack <= 1) {
-    f(IntC<1>{});
-  } else if (npack <= 2) {
+  if (npack <= 2) {
     f(IntC<2>{});
   } else if (npack <= 4) {
     f(IntC<4>{});
@@ -480,27 +475,27 @@ int launch_typed(void* out, const void* x, const void* res, void* res_out, const
     return check_launch("rms_norm kernel launch");
   }
   if (packs <= kRowsMaxPacks) {
-    auto rows_kernel = [&](auto lanes, auto np) {
-      constexpr int L = decltype(lanes)::value, NP = decltype(np)::value;
+    auto rows_kernel = [&](auto lanes) {
+      constexpr int L = decltype(lanes)::value;
       const unsigned wgs = static_cast<unsigned>(cdiv(rows, kRowsThreads / L));
       if (aligned) {
-        rms_norm_rows_kernel<E, L, NP, HAS_RES, true><<<wgs, kRowsThreads, 0, stream>>>(
+        rms_norm_rows_kernel<E, L, HAS_RES, true><<<wgs, kRowsThreads, 0, stream>>>(
             o, xi, r, rw, wi, static_cast<int>(rows), hidden, xm, eps);
       } else {
-        rms_norm_rows_kernel<E, L, NP, HAS_RES, false><<<wgs, kRowsThreads, 0, stream>>>(
+        rms_norm_rows_kernel<E, L, HAS_RES, false><<<wgs, kRowsThreads, 0, stream>>>(
             o, xi, r, rw, wi, static_cast<int>(rows), hidden, xm, eps);
       }
     };
     if (packs <= 4) {
-      rows_kernel(IntC<4>{}, IntC<1>{});
+      rows_kernel(IntC<4>{});
     } else if (packs <= 8) {
-      rows_kernel(IntC<8>{}, IntC<1>{});
+      rows_kernel(IntC<8>{});
     } else if (packs <= 16) {
-      rows_kernel(IntC<16>{}, IntC<1>{});
+      rows_kernel(IntC<16>{});
     } else if (packs <= 32) {
-      rows_kernel(IntC<32>{}, IntC<1>{});
+      rows_kernel(IntC<32>{});
     } else {
-      rows_kernel(IntC<64>{}, IntC<1>{});
+      rows_kernel(IntC<64>{});
     }
     return check_launch("rms_norm kernel launch");
   }
