@@ -204,7 +204,7 @@ def test_planner_pairs_long_contexts_of_small_batches(batch, hkv, max_pages, pai
 
 def test_requested_balanced_schedule_at_any_batch():
     """KL_SPLITS_BALANCED (-1) picks the balanced schedule whatever the planner
-    default; the VALU path (fp32) takes the planner's uniform splits."""
+    default; fp32 takes the planner's uniform splits."""
     with _native.decode_switches(balance_always="0"):
         assert ops.plan_decode(torch.float16, 64, 32, 8, 128, 16, 256, 0, 256)[0] == 1
         splits, ws = ops.plan_decode(torch.float16, 64, 32, 8, 128, 16, 256, ops.BALANCED, 256)

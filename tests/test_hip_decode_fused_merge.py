@@ -197,3 +197,68 @@ def test_fresh_partials_every_call(gpu_ops, lens, splits):
         fused = _decode(gpu_ops, q, kv, **kw)
         merged = _unfused(lambda: _decode(gpu_ops, q, kv, **kw))
         assert torch.equal(fused, merged), f"call {i}: fused merge differs from the merge kernel"
+
+
+F32, BF16 = torch.float32, torch.bfloat16
+
+
+@pytest.mark.parametrize(
+    ("cache", "lens", "hq", "hkv", "head_dim", "page", "num_splits", "merge"),
+    [
+        (F32, [2000, 0, 1500, 17, 700, 2000, 1, 900], 32, 8, 128, 16, None, IN_KERNEL),  # eight waves, four splits
+        (F32, [1500, 0, 40], 16, 4, 256, 16, None, IN_KERNEL),  # four waves
+        (F32, [900, 0, 33, 600], 8, 8, 64, 48, 5, IN_KERNEL),
+        (F32, [900, 0, 33, 600], 32, 1, 128, 16, 4, MERGE_KERNEL),  # two head tiles
+        (F32, [900, 0, 33, 600], 16, 4, 128, 5, 3, IN_KERNEL),  # small pages
+        (BF16, [2000, 0, 1500, 17, 700, 2000, 1, 900], 32, 8, 128, 8, None, IN_KERNEL),  # small pages, balanced
+        (BF16, [1000, 0, 500, 17, 700, 999, 1, 900], 32, 8, 128, 8, None, IN_KERNEL),  # small pages, uniform splits
+        (BF16, [900, 0, 33, 600], 8, 4, 256, 1, 7, IN_KERNEL),
+        ("fp8", [2000, 0, 1500, 17], 16, 4, 128, 16, None, IN_KERNEL),  # balanced, eight waves
+        ("fp8", [6000, 0, 1500, 17], 32, 1, 128, 16, None, MERGE_KERNEL),  # the same with two head tiles
+    ],
+)
+def test_fused_merge_of_other_caches(gpu_ops, cache, lens, hq, hkv, head_dim, page, num_splits, merge):
+    """fp32, small-page and eight-wave FP8 units merge in the kernel too, with the
+    merge kernel's bits."""
+    dtype = BF16 if cache == "fp8" else cache
+    q, kv, _, _ = random_decode_problem([max(n, 1) for n in lens], hq, hkv, head_dim, page, dtype=dtype, device="cuda",
+                                        poison=float("nan"), seed=page + hq)
+    scales = {}
+    if cache == "fp8":
+        kv, scales["k_scale"], scales["v_scale"] = quantize_fp8(kv)
+    kv.seq_lens = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    run = lambda: _decode(gpu_ops, q, kv, num_splits=num_splits, **scales).cpu()  # noqa: E731
+    fused = run()
+    assert _last_merge() == merge, "the call did not take the expected merge"
+    merged = _unfused(run)
+    assert _last_merge() == MERGE_KERNEL
+    assert torch.equal(fused, merged), "fused merge differs from the merge kernel"
+    assert not fused[1].any(), "an empty sequence must give zeros"
+    rows = [b for b, n in enumerate(lens) if n]
+    args = (q[rows].cpu().float(), kv.k_cache.cpu(), kv.v_cache.cpu(), kv.block_table[rows].cpu(), kv.seq_lens[rows].cpu())
+    if cache == "fp8":
+        want = ref.paged_decode_attention_fp8(*args, scales["k_scale"].cpu(), scales["v_scale"].cpu())
+    else:
+        want = ref.paged_decode_attention(*args)
+    decode_parity(fused[rows], want, dtype)
+
+
+@pytest.mark.parametrize("page", [16, 8])
+def test_concurrent_streams_fp32(gpu_ops, page):
+    jobs = []
+    for i in range(4):
+        q, kv = device_decode_problem([1500] * 6, 32, 8, 128, page, dtype=F32, seed=80 + i)
+        want = _unfused(lambda q=q, kv=kv: _decode(gpu_ops, q, kv)).clone()
+        jobs.append((torch.cuda.Stream(), q, kv, torch.empty_like(q), want))
+    torch.cuda.synchronize()
+    for _ in range(3):
+        for stream, q, kv, out, _ in jobs:
+            stream.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(stream):
+                for _ in range(4):
+                    _decode(gpu_ops, q, kv, out=out)
+        torch.cuda.synchronize()
+        for i, (_, _, _, out, want) in enumerate(jobs):
+            assert torch.equal(out, want), f"stream {i}"
+            out.zero_()
+        torch.cuda.synchronize()
