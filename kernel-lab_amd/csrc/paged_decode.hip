@@ -2418,10 +2418,10 @@ __global__ void __launch_bounds__(64) decode_merge_balanced_kernel(const DecodeA
 // holds two workgroups, and short ones make room for the next. What is left is
 // the two workgroups a CU runs one after the other, each a chain of blocks.
 // Measured, a launch per pass -> this, merge included (us): 32/8/128 fp16 B=64
-// prefix 4,096 own up to 1,024 55.1 -> 49.6, B=32 16,384 + 256 44.6 -> 39.1,
+// prefix 4,096 own up to 1,024 54.3 -> 48.9, B=32 16,384 + 256 44.6 -> 39.1,
 // 64/8/128 bf16 B=16 16,384 + 1,024 47.9 -> 44.4, 32/8/128 B=4 2,000 + 300 18.5
-// -> 13.7. The own tokens first: 54.6; twice the prefix splits: 50.6; own
-// splits of 32 pages: 51.8. NTP, NTS: head tiles of the two passes.
+// -> 13.7. At the first shape, on another day at 49.6: the own tokens first 54.6,
+// twice the prefix splits 50.6, own splits of 32 pages 51.8. NTP, NTS: head tiles of the two passes.
 //
 // This launch has no KV-head pairs: with 8-wave workgroups a CU would hold one.
 // Where the own pass pairs (a full batch) and streams long sequences, pairs are

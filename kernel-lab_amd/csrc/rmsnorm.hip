@@ -59,7 +59,8 @@ constexpr int kMaxThreads = 1024;
 // row_stride, inner rows to a group; out and the residuals hold row g * inner +
 // i there. A strided view of two leading dimensions (the heads of one part of a
 // fused projection) is read in place; copied first, 2,048 x 32 heads of 128
-// bf16 took 15.7 us, the copy 9.7 of them, and 7.1 read in place.
+// bf16 took 15.7 us a call, the copy 9.7 of them, and 6.9 read in place (calls back
+// to back; the kernel alone traces at 7.3 with the profiler's gaps).
 //
 // A workgroup per row takes (i, g) from the grid, the larger of the two counts
 // along x: a division before the first load cost the large sizes 2 %.
