@@ -2952,7 +2952,8 @@ int make_plan(const Options& opt, kl_dtype dtype, int batch, int num_q_heads, in
   // ctx 512 11.24 -> 9.92, ctx 4096 16.28 -> 13.20, ctx 32768 33.04 -> 31.76;
   // 8/1/128 ctx 32768 26.08 -> 16.40.
   const bool single = batch == 1 && !long_pairs;
-  const bool short_units = !whole_blocks && table_tokens <= kUniformSmallPageTokens;
+  const bool short_units =
+      !whole_blocks && table_tokens <= kUniformSmallPageTokens && full_batch_choice != 1;
   const bool automatic =
       num_splits == 0 && !single && !short_units && list_fits &&
       (units < cus || (full_batch_choice < 0 ? full_default : full_batch_choice == 1));

@@ -275,6 +275,8 @@ def test_short_small_page_tables_take_uniform_splits(batch, tokens, splits):
     """Pages of 8 tokens: tables of up to 1,024 tokens take uniform splits (of at
     least 16 blocks of 16 tokens), longer ones the balanced schedule (0)."""
     assert ops.plan_decode(torch.float16, batch, 32, 8, 128, 8, tokens // 8, 0, 256)[0] == splits
+    with _native.decode_switches(balance_always="1"):
+        assert ops.plan_decode(torch.float16, batch, 32, 8, 128, 8, tokens // 8, 0, 256)[0] == 0
 
 
 def test_planner_rejects_bad_shapes():
