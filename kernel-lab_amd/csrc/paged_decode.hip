@@ -489,7 +489,7 @@ __device__ __forceinline__ void load_q(const DecodeArgs& a, const Unit& u, QFrag
     const S* qh = q + q_row(a, u, hl < a.group ? hl : 0) * D;
 #pragma unroll
     for (int c = 0; c < qk_chunks<E, D>(); ++c) {
-      qf.v[t][c] = *reinterpret_cast<const u32x4*>(qh + EPC * (4 * c + grp));
+      qf.v[t][c] = *reinterpret_cast<const u32x4*>(qh + 4 * EPC * c + EPC * grp);
     }
   }
 }
@@ -811,8 +811,23 @@ __device__ __forceinline__ void mfma_segment(const DecodeArgs& a, char* lds, con
     }
   };
   auto load_block = [&](const auto& src, u32x4 (&kf)[NL], u32x4 (&vf)[NL], bool live) {
-    load_half(kc, src, kf, live);
-    load_half(vc, src, vf, live);
+    if constexpr (SP) {
+      load_half(kc, src, kf, live);
+      load_half(vc, src, vf, live);
+    } else {
+      // Both resources before the first load: built between the halves they cost
+      // the register pipeline 1 % on short launches (8/1/64 fp16 B=10 of 95 tokens
+      // 21.5 -> 21.7 us).
+      const int records = live ? 0x7fffffff : 0;
+      const auto kr = __builtin_amdgcn_make_buffer_rsrc(const_cast<KS*>(kc + src), static_cast<short>(0), records,
+                                                        kBufferDword3);
+      const auto vr = __builtin_amdgcn_make_buffer_rsrc(const_cast<KS*>(vc + src), static_cast<short>(0), records,
+                                                        kBufferDword3);
+#pragma unroll
+      for (int c = 0; c < NL; ++c) kf[c] = buffer_load16<kKvPolicy>(kr, kv_off[c]);
+#pragma unroll
+      for (int c = 0; c < NL; ++c) vf[c] = buffer_load16<kKvPolicy>(vr, kv_off[c]);
+    }
   };
   // One 16-byte load's elements into a staging row as E: a plain store for a
   // 16-bit cache, decoded to two 16-byte chunks for FP8.
